@@ -92,10 +92,11 @@ struct SchurWork {
 	int *status = nullptr;
 };
 
-// Buffers of the stabilised slice product (allocated on first use): U, V, the QR work matrix and
-// X (N x N each), the column scales d, reflector factors tau, the column order, the reflector count.
+// Buffers of the stabilised slice product (allocated on first use): U, the two buffers V alternates
+// between, the QR work matrix (N x N each), the column scales d and sort keys, the panels' T factors,
+// inverse diagonal blocks of R and reflectors, the column order, the reflector counts of U and of X.
 struct StabWork {
-	double *U = nullptr, *V = nullptr, *ZR = nullptr, *X = nullptr, *d = nullptr, *tau = nullptr;
+	double *U = nullptr, *V[2] = {nullptr, nullptr}, *ZR = nullptr, *d = nullptr, *key = nullptr, *T = nullptr, *Rinv = nullptr, *Vm = nullptr;
 	int *perm = nullptr, *nref = nullptr;
 };
 

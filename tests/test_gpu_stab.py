@@ -115,3 +115,23 @@ def test_chain_with_stabilize_takes_the_plain_decisions(precision):
         say("traj %d: plain dH %.6g acc %d, stabilised dH %.6g acc %d" % (it, a.dH, a.accepted, b.dH, b.accepted))
         assert a.accepted == b.accepted, it
         assert b.logdet == pytest.approx(a.logdet, rel=tol), it
+
+
+# sizes at the edges of the QR's panels (32 columns, 16 above 1024 sites), of its workgroup shapes
+# (128, 256, 512 rows) and of its 16- and 64-row tiles
+@pytest.mark.parametrize("l1,l2,nt,k", [(1, 1, 4, 1), (5, 5, 8, 3), (4, 8, 8, 8), (3, 11, 9, 2), (8, 16, 8, 3), (3, 43, 8, 4),
+                                        (16, 16, 8, 8), (257, 1, 8, 4), (16, 32, 8, 4), (27, 19, 8, 8), (32, 32, 8, 4),
+                                        (41, 25, 8, 4)])
+def test_blocked_qr_sizes(l1, l2, nt, k):
+    """Log det and inverse against numpy's for the plain product at beta = 4, where it is well
+    conditioned (each element's relative error is a few hundred eps: 1e-11 leaves a factor of 100)."""
+    om = OracleModel(l1, l2, nt, beta=4.0)
+    ctx = gpu_context(om)
+    x = np.random.default_rng(l1 + l2).standard_normal(om.dim)
+    n = l1 * l2
+    say("blocked QR", l1, l2, nt, k)
+    M = ctx.M_hat(x).reshape(n, n).T
+    sign, ld = np.linalg.slogdet(M)
+    ld1, s1, inv1 = ctx.stable_logdet_inv(x, 0, k)
+    assert s1 == sign and ld1 == pytest.approx(ld, rel=1e-11)
+    assert rel(inv1, np.linalg.inv(M).T.ravel()) < 1e-11
