@@ -115,11 +115,24 @@ __device__ void reduce_links(const P *__restrict__ part, unsigned nwg, unsigned 
 template <typename R, int C>
 constexpr bool adj_lean(){ return C * sizeof(R) <= 16; }
 
+// Place of value (site, c) in an LDS buffer of np sites: the C columns in planes of the widest read
+// (16 bytes), each [site][column].  One plane up to 16 bytes per site; fp64 at 4 columns takes two: a
+// 32-byte stride between sites would put lanes 8 apart on the same banks in every read.
+template <typename R, int C>
+__host__ __device__ constexpr int adj_vec(){ return C * sizeof(R) <= 16 ? C : 16 / (int)sizeof(R); }
+
+template <typename R, int C>
+__device__ __forceinline__ size_t adj_at(unsigned site, int c, unsigned np)
+{
+	constexpr int V = adj_vec<R, C>();
+	return V == C ? (size_t)site * C + c : (size_t)(c / V) * np * V + (size_t)site * V + c % V;
+}
+
 // BATCH: the six neighbour reads are issued before any of them is used; otherwise each is read
 // just before its sums, which holds fewer registers. The sum is taken in the order d = 0..5
 // either way.
 template <typename R, int C, bool BATCH>
-__device__ __forceinline__ void gather6(const R *__restrict__ buf, const int (&nbr)[6], const R (&cf)[6], R mu,
+__device__ __forceinline__ void gather6(const R *__restrict__ buf, unsigned np, const int (&nbr)[6], const R (&cf)[6], R mu,
 		const R (&own)[C], R (&out)[C])
 {
 #pragma unroll
@@ -129,7 +142,7 @@ __device__ __forceinline__ void gather6(const R *__restrict__ buf, const int (&n
 #pragma unroll
 		for(int d = 0; d < 6; d++)
 #pragma unroll
-			for(int c = 0; c < C; c++) nv[d][c] = buf[(size_t)nbr[d] * C + c];
+			for(int c = 0; c < C; c++) nv[d][c] = buf[adj_at<R, C>(nbr[d], c, np)];
 #pragma unroll
 		for(int d = 0; d < 6; d++)
 #pragma unroll
@@ -137,9 +150,8 @@ __device__ __forceinline__ void gather6(const R *__restrict__ buf, const int (&n
 	}else{
 #pragma unroll
 		for(int d = 0; d < 6; d++){
-			const R *q = buf + (size_t)nbr[d] * C;
 #pragma unroll
-			for(int c = 0; c < C; c++) out[c] = fmac(cf[d], q[c], out[c]);
+			for(int c = 0; c < C; c++) out[c] = fmac(cf[d], buf[adj_at<R, C>(nbr[d], c, np)], out[c]);
 		}
 	}
 }
@@ -229,23 +241,23 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 				for(int j = 0; j < S; j++)
 					if(act[j])
 #pragma unroll
-						for(int c = 0; c < C; c++) buf0[(size_t)site[j] * C + c] = v[j][c];
+						for(int c = 0; c < C; c++) buf0[adj_at<R, C>(site[j], c, ns)] = v[j][c];
 				__syncthreads();
 #pragma unroll
 				for(int j = 0; j < S; j++)
-					if(act[j]) gather6<R, C, BATCH>(buf0, nbr[j], cf[j], a.mu, v[j], w[j]);
+					if(act[j]) gather6<R, C, BATCH>(buf0, ns, nbr[j], cf[j], a.mu, v[j], w[j]);
 				if(a.cplx[p]){
 #pragma unroll
 					for(int j = 0; j < S; j++)
 						if(act[j])
 #pragma unroll
-							for(int c = 0; c < C; c++) buf1[(size_t)site[j] * C + c] = w[j][c];
+							for(int c = 0; c < C; c++) buf1[adj_at<R, C>(site[j], c, ns)] = w[j][c];
 					__syncthreads();
 #pragma unroll
 					for(int j = 0; j < S; j++){
 						if(!act[j]) continue;
 						R z[C];
-						gather6<R, C, BATCH>(buf1, nbr[j], cf[j], a.mu, w[j], z);
+						gather6<R, C, BATCH>(buf1, ns, nbr[j], cf[j], a.mu, w[j], z);
 #pragma unroll
 						for(int c = 0; c < C; c++) v[j][c] = v[j][c] + fmac(a.a_quad[p], z[c], a.a_lin[p] * w[j][c]);
 					}
@@ -327,7 +339,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 		for(int j = 0; j < S; j++)
 			if(act[j])
 #pragma unroll
-				for(int c = 0; c < C; c++) wbs[0][(size_t)site[j] * C + c] = wv[j][c];
+				for(int c = 0; c < C; c++) wbs[0][adj_at<R, C>(site[j], c, ns)] = wv[j][c];
 	};
 	if(a.w0_early) put_w0();
 	load_slice(a.tau_e - 1);
@@ -359,7 +371,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 			for(int j = 0; j < S; j++)
 				if(act[j])
 #pragma unroll
-					for(int c = 0; c < C; c++) bb[(size_t)site[j] * C + c] = t[j][c];
+					for(int c = 0; c < C; c++) bb[adj_at<R, C>(site[j], c, ns)] = t[j][c];
 			__syncthreads();
 			if(FOLD && a.w0_early && b == 1 && tau_out >= 0) flush_bonds();
 #pragma unroll
@@ -367,7 +379,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 				// with ALL_LANES a thread past the last site gathers too (neighbour 0, in bounds)
 				// and stores nothing
 				R tn[C];
-				if(ALL_LANES || act[j]) gather6<R, C, BATCH>(bb, nbr[j], cf[j], a.mu, t[j], tn);
+				if(ALL_LANES || act[j]) gather6<R, C, BATCH>(bb, ns, nbr[j], cf[j], a.mu, t[j], tn);
 				else
 #pragma unroll
 					for(int c = 0; c < C; c++) tn[c] = 0;
@@ -406,7 +418,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 				for(int j = 0; j < S; j++)
 					if(act[j])
 #pragma unroll
-						for(int c = 0; c < C; c++) wb[(size_t)site[j] * C + c] = wa[j][c];
+						for(int c = 0; c < C; c++) wb[adj_at<R, C>(site[j], c, ns)] = wa[j][c];
 				__syncthreads();
 				if(FOLD && !a.w0_early && q == 0 && tau_out >= 0) flush_bonds();
 			}
@@ -422,7 +434,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 #pragma unroll
 					for(int d = 0; d < 6; d++)
 #pragma unroll
-						for(int c = 0; c < C; c++) nv[d][c] = wb[(size_t)nbr[j][d] * C + c];
+						for(int c = 0; c < C; c++) nv[d][c] = wb[adj_at<R, C>(nbr[j][d], c, ns)];
 				}
 #pragma unroll
 				for(int c = 0; c < C; c++) wn[c] = a.mu * wa[j][c];
@@ -431,7 +443,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 					const int dv = NV == 6 ? d : 0;
 					if constexpr(NV == 1){
 #pragma unroll
-						for(int c = 0; c < C; c++) nv[0][c] = wb[(size_t)nbr[j][d] * C + c];
+						for(int c = 0; c < C; c++) nv[0][c] = wb[adj_at<R, C>(nbr[j][d], c, ns)];
 					}
 					R hs = 0;
 #pragma unroll

@@ -13,6 +13,8 @@
 // forward bonds, including lattices of extent 1 or 2 where bonds alias.
 #include "internal.h"
 #include "stencil.h"
+#include "patch.h"
+#include <vector>
 #include <cstdlib>
 #include <algorithm>
 #include <cstring>
@@ -61,12 +63,48 @@ __global__ void coef_multi_kernel(const CoefArgs *__restrict__ tab)
 	coef_body(a.x, a.link, a.t[0], a.t[1], a.t[2], a.k[0], a.k[1], a.k[2], a.ns, a.nt, a.c64, a.c32, blockIdx.x, a.gx);
 }
 
+// the site form's coefficients (blockIdx.y < nt: slice blockIdx.y) and the patch form's
+// (blockIdx.y - nt: its slice) of one arithmetic, in one launch
+template <typename R>
+__global__ __launch_bounds__(256) void coef_patch_kernel(const double *__restrict__ x, const unsigned *__restrict__ link,
+		double t0, double t1, double t2, double k0, double k1, double k2, unsigned ns, unsigned nt, double *__restrict__ c64,
+		float *__restrict__ c32, const int *__restrict__ bond, unsigned nbond, R *__restrict__ out)
+{
+	const bool site = blockIdx.y < nt;
+	const size_t tau = site ? blockIdx.y : blockIdx.y - nt;
+	const unsigned n = site ? 6 * ns : nbond;
+	for(unsigned e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256){
+		const int b = site ? (int)link[e] : bond[e], k = b % 3;
+		const double tk = k == 0 ? t0 : (k == 1 ? t1 : t2);
+		const double kk = k == 0 ? k0 : (k == 1 ? k1 : k2);
+		const double f = tk - kk * x[tau * 3 * ns + b];
+		if(site){
+			c64[tau * n + e] = f;
+			if(c32) c32[tau * n + e] = (float)f;
+		}else out[tau * n + e] = (R)f;
+	}
+}
+
 int coefficients(ephmc_ctx *c, const double *x, bool want32)
 {
+	const double *t = c->cfg.t, *k = c->cfg.kappa;
+	float *c32 = want32 ? c->d_coef32 : nullptr;
+	const PatchTab &pt = c->patch[want32 ? 1 : 0];
+	c->patch_slot = -1;
+	if(patch_on(c, want32 ? EPHMC_MIXED : EPHMC_FP64)){
+		c->patch_slot = want32 ? 1 : 0;
+		const unsigned m = pt.nk * pt.tp;
+		const dim3 g((std::max(m, 6 * c->ns) + 255) / 256, 2 * c->nt);
+		if(want32) coef_patch_kernel<float><<<g, 256, 0, c->stream>>>(x, c->d_link, t[0], t[1], t[2], k[0], k[1], k[2], c->ns, c->nt,
+			c->d_coef64, c32, pt.bond, m, (float *)pt.coef);
+		else coef_patch_kernel<double><<<g, 256, 0, c->stream>>>(x, c->d_link, t[0], t[1], t[2], k[0], k[1], k[2], c->ns, c->nt,
+			c->d_coef64, c32, pt.bond, m, (double *)pt.coef);
+		EPHMC_LAUNCHED();
+		return EPHMC_OK;
+	}
 	const size_t n = (size_t)c->nt * 6 * c->ns;
 	const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 4096);
-	coef_kernel<<<blocks, 256, 0, c->stream>>>(x, c->d_link, c->cfg.t[0], c->cfg.t[1], c->cfg.t[2],
-		c->cfg.kappa[0], c->cfg.kappa[1], c->cfg.kappa[2], c->ns, c->nt, c->d_coef64, want32 ? c->d_coef32 : nullptr);
+	coef_kernel<<<blocks, 256, 0, c->stream>>>(x, c->d_link, t[0], t[1], t[2], k[0], k[1], k[2], c->ns, c->nt, c->d_coef64, c32);
 	EPHMC_LAUNCHED();
 	return EPHMC_OK;
 }
@@ -331,6 +369,249 @@ __global__ __launch_bounds__(LB) void chain_strip_kernel(ChainArgs<R> a)
 	}
 }
 
+// ---------------------------------------------------------------------------------------------
+// Patch form of the same chain (patch.h): a thread owns PX x PY sites of C columns, a workgroup all
+// patches of them.  Up to 64 patches are one wave, and its steps need no barrier.  The bonds of the
+// next slice are loaded during the current one, except above 512 threads, where the registers for
+// them would spill.
+//
+// What bounds it: LDS reads plus vector issue, which overlap little, as a barrier between any two
+// stencils keeps the waves in step.  Against the site form a 2 x 2 patch reads 10 neighbours
+// per 4 sites instead of 24, without the bank conflicts of the strip form's consecutive sites, and each
+// bond once instead of twice.  us per chain (chain kernel and coefficients), before -> now:
+// fp64 6x6 nt 32 38 -> 31, 16x16 nt 64 79 -> 67, 21x19 nt 95 165 -> 141, 27x31 nt 64 325 -> 224,
+// 32x32 nt 128 545 -> 433, 64x32 nt 32 1041 -> 548; fp32 21x19 118 -> 111, 24x24 nt 64 178 -> 105,
+// 32x32 301 -> 271, 36x36 nt 32 250 -> 156, 45x45 410 -> 354.
+template <typename R>
+struct PatchArgs {
+	const R *coef;          // [nt][bonds][tp]
+	const int *halo;        // [halo][tp]: LDS places of the halo sites
+	R mu;
+	unsigned ns, l1, l2, npx, np, tp;     // patches per row, patches, places per slot
+	const R *src;
+	R *dst, *ck;
+	unsigned ck_every;
+	int tau0, dir, ntau, npairs;
+	R a_lin[MAX_PAIRS], a_quad[MAX_PAIRS];
+};
+
+template <typename R, int C, int PX, int PY, int LB>
+__global__ __launch_bounds__(LB) void chain_patch_kernel(PatchArgs<R> a)
+{
+	extern __shared__ __align__(16) unsigned char smem_raw[];
+	constexpr int S = PX * PY, NH = patch_halo(PX, PY), NK = patch_bonds(PX, PY);
+	constexpr bool AHEAD = LB <= 512;
+	struct alignas(C * sizeof(R) <= 16 ? C * sizeof(R) : 16) Vec { R v[C]; };
+	const unsigned tp = a.tp, ns = a.ns, col0 = blockIdx.x * C;
+	Vec *V = reinterpret_cast<Vec *>(smem_raw), *W = V + (size_t)S * tp;
+	// a thread past the last patch works on it too (the same values, to the same LDS places) and
+	// stores nothing
+	const bool act = threadIdx.x < a.np;
+	const unsigned p = act ? threadIdx.x : a.np - 1;
+	const unsigned x0 = p % a.npx * PX, y0 = p / a.npx * PY;
+	int halo[NH];
+#pragma unroll
+	for(int k = 0; k < NH; k++) halo[k] = a.halo[(size_t)k * tp + p];
+	R v[S][C], cf[NK], cn[NK];
+	// (x, y) of this patch: its column-major place, and whether this patch owns the site
+	auto place = [&](int x, int y){ return (y0 + y) % a.l2 * a.l1 + (x0 + x) % a.l1; };
+	auto owns = [&](int x, int y){ return act && x0 + x < a.l1 && y0 + y < a.l2; };
+#pragma unroll
+	for(int s = 0; s < S; s++){
+		const unsigned site = place(s % PX, s / PX);
+#pragma unroll
+		for(int c = 0; c < C; c++){
+			const unsigned col = col0 + c;
+			v[s][c] = 0;
+			if(col < ns) v[s][c] = a.src ? a.src[(size_t)col * ns + site] : (R)(site == col ? 1 : 0);
+		}
+	}
+	auto store = [&](R *m){
+#pragma unroll
+		for(int c = 0; c < C; c++){
+			if(col0 + c >= ns) break;
+			R *q = m + (size_t)(col0 + c) * ns;
+#pragma unroll
+			for(int s = 0; s < S; s++)
+				if(owns(s % PX, s / PX)) q[(y0 + s / PX) * a.l1 + x0 + s % PX] = v[s][c];
+		}
+	};
+	auto load_bonds = [&](int i){
+		const R *q = a.coef + (size_t)(a.tau0 + a.dir * i) * NK * tp + p;
+#pragma unroll
+		for(int k = 0; k < NK; k++) cn[k] = q[(size_t)k * tp];
+	};
+	auto apply = [&](Vec *buf, const R (&in)[S][C], R (&out)[S][C]){
+#pragma unroll
+		for(int s = 0; s < S; s++){
+			Vec t;
+#pragma unroll
+			for(int c = 0; c < C; c++) t.v[c] = in[s][c];
+			buf[s * tp + p] = t;
+		}
+		__syncthreads();
+		R h[NH][C];
+#pragma unroll
+		for(int k = 0; k < NH; k++){
+			const Vec t = buf[halo[k]];
+#pragma unroll
+			for(int c = 0; c < C; c++) h[k][c] = t.v[c];
+		}
+		patch_stencil<R, C, PX, PY>(in, h, cf, a.mu, out);
+	};
+	if(AHEAD && a.ntau > 0) load_bonds(0);
+	for(int i = 0; i < a.ntau; i++){
+		if(!AHEAD) load_bonds(i);
+		if(a.ck && (i % a.ck_every) == 0) store(a.ck + (size_t)(i / a.ck_every) * ns * ns);
+#pragma unroll
+		for(int k = 0; k < NK; k++) cf[k] = cn[k];
+		if(AHEAD && i + 1 < a.ntau) load_bonds(i + 1);
+#pragma unroll 1
+		for(int q = 0; q < a.npairs; q++){
+			// V is free: its last readers passed the barrier of the pair's second stencil, and W's
+			// passed the barrier of the next first one
+			R w[S][C], z[S][C];
+			apply(V, v, w);
+			apply(W, w, z);
+#pragma unroll
+			for(int s = 0; s < S; s++)
+#pragma unroll
+				for(int c = 0; c < C; c++) v[s][c] = v[s][c] + fmac(a.a_quad[q], z[s][c], a.a_lin[q] * w[s][c]);
+		}
+	}
+	if(a.dst) store(a.dst);
+}
+
+template <typename R>
+static PatchArgs<R> patch_args(const ephmc_ctx *c, const PatchTab &t)
+{
+	PatchArgs<R> a{};
+	a.coef = (const R *)t.coef;
+	a.halo = t.halo;
+	a.mu = (R)c->cfg.mu;
+	a.ns = c->ns;
+	a.l1 = c->l1;
+	a.l2 = c->l2;
+	a.npx = t.npx;
+	a.np = t.np;
+	a.tp = t.tp;
+	a.npairs = c->poly.np;
+	for(int p = 0; p < c->poly.np; p++){
+		a.a_lin[p] = (R)c->poly.a_lin[p];
+		a.a_quad[p] = (R)c->poly.a_quad[p];
+	}
+	return a;
+}
+
+template <typename R, int C, int PX, int PY>
+static int launch_patch_lb(ephmc_ctx *c, const PatchArgs<R> &a)
+{
+	const size_t lds = 2 * (size_t)C * PX * PY * a.tp * sizeof(R);
+	if(lds > 160 * 1024 || a.tp > 1024){ set_error("chain: %zu B of LDS, %u threads", lds, a.tp); return EPHMC_ERR_ARG; }
+	const unsigned blocks = (a.ns + C - 1) / C;
+#define EPHMC_PATCH_LAUNCH(LB)                                                                          \
+	do {                                                                                                \
+		(void)hipFuncSetAttribute((const void *)chain_patch_kernel<R, C, PX, PY, LB>,                    \
+			hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                                       \
+		chain_patch_kernel<R, C, PX, PY, LB><<<blocks, a.tp, lds, c->stream>>>(a);                       \
+	} while(0)
+	if(a.tp <= 64) EPHMC_PATCH_LAUNCH(64);
+	else if(a.tp <= 256) EPHMC_PATCH_LAUNCH(256);
+	else if(a.tp <= 512) EPHMC_PATCH_LAUNCH(512);
+	else if(a.tp <= 640) EPHMC_PATCH_LAUNCH(640);
+	else EPHMC_PATCH_LAUNCH(1024);
+#undef EPHMC_PATCH_LAUNCH
+	EPHMC_LAUNCHED();
+	return EPHMC_OK;
+}
+
+template <typename R>
+static int launch_patch(ephmc_ctx *c, const PatchTab &t, PatchArgs<R> a)
+{
+#define EPHMC_PATCH(CC, X, Y) if(t.cols == CC && t.px == X && t.py == Y) return launch_patch_lb<R, CC, X, Y>(c, a)
+	EPHMC_PATCH(1, 1, 1);
+	EPHMC_PATCH(2, 1, 1);
+	EPHMC_PATCH(2, 2, 2);
+#undef EPHMC_PATCH
+	set_error("chain: no patch form for %u columns of %u x %u sites", t.cols, t.px, t.py);
+	return EPHMC_ERR_ARG;
+}
+
+// Tables of the patch form for one arithmetic, where it is the faster form of the chain (measured
+// shapes above): fp64 up to 512 sites one site per thread and one column per workgroup, above 640
+// sites 2 x 2 sites and 2 columns (between, the strip form by 3 % where l1 is even); fp32 not up to
+// 256 sites (16x16 nt 64: 62 against 55 us for the site form), one site and 2 columns up to 640, 2 x 2
+// sites and 2 columns beyond.
+int patch_reserve(ephmc_ctx *c, int prec)
+{
+	PatchTab &t = c->patch[prec == EPHMC_FP64 ? 0 : 1];
+	const unsigned ns = c->ns;
+	if(prec != EPHMC_FP64 && ns <= 256) return EPHMC_OK;
+	if(prec == EPHMC_FP64 && ns > 512 && ns <= 640 && c->l1 % 2 == 0) return EPHMC_OK;
+	const unsigned X = ns <= 640 ? 1 : 2, Y = X;
+	t.cols = prec == EPHMC_FP64 && ns <= 640 ? 1 : 2;
+	t.px = X; t.py = Y;
+	t.npx = (c->l1 + X - 1) / X;
+	t.np = t.npx * ((c->l2 + Y - 1) / Y);
+	t.tp = (t.np + 63) / 64 * 64;
+	if(t.tp > 1024){ t = PatchTab{}; return EPHMC_OK; }        // (long thin lattices)
+	t.nk = patch_bonds(X, Y);
+	const unsigned nh = patch_halo(X, Y), tp = t.tp;
+	std::vector<int> tab((size_t)(nh + t.nk) * tp, 0);
+	int *halo = tab.data(), *bond = halo + (size_t)nh * tp;
+	for(unsigned p = 0; p < tp; p++){
+		const unsigned q = std::min(p, t.np - 1);
+		const int x0 = (int)(q % t.npx * X), y0 = (int)(q / t.npx * Y), l1 = (int)c->l1, l2 = (int)c->l2;
+		auto wrap = [](int v, int l){ return (v % l + l) % l; };
+		auto place = [&](int x, int y){
+			const unsigned xs = wrap(x0 + x, l1), ys = wrap(y0 + y, l2);
+			return (int)((ys % Y * X + xs % X) * tp + ys / Y * t.npx + xs / X);
+		};
+		auto link = [&](int x, int y, int k){ return 3 * (wrap(y0 + y, l2) * l1 + wrap(x0 + x, l1)) + k; };
+		unsigned h = 0, b = 0;
+		auto put = [&](int x, int y){ halo[(size_t)h++ * tp + p] = place(x, y); };
+		auto bnd = [&](int x, int y, int k){ bond[(size_t)b++ * tp + p] = link(x, y, k); };
+		for(int x = 0; x <= (int)X; x++) put(x - 1, Y);
+		for(int x = 0; x <= (int)X; x++) put(x, -1);
+		for(int y = 0; y < (int)Y; y++) put(-1, y);
+		for(int y = 0; y < (int)Y; y++) put(X, y);
+		for(int y = 0; y < (int)Y; y++) for(int x = 0; x < (int)X; x++) for(int k = 0; k < 3; k++) bnd(x, y, k);
+		for(int y = 0; y < (int)Y; y++) bnd(-1, y, 0);
+		for(int x = 0; x < (int)X; x++) bnd(x, -1, 1);
+		for(int x = 0; x < (int)X; x++) bnd(x + 1, -1, 2);
+		for(int y = 0; y + 1 < (int)Y; y++) bnd(X, y, 2);
+	}
+	// one allocation: the coefficients, then both tables
+	const size_t csz = (size_t)c->nt * t.nk * tp * (prec == EPHMC_FP64 ? 8 : 4), tsz = tab.size() * sizeof(int);
+	if(hipMalloc(&t.coef, csz + tsz) != hipSuccess){
+		(void)hipGetLastError();
+		t = PatchTab{};
+		set_error("patch tables (%zu bytes) could not be allocated", csz + tsz);
+		return EPHMC_ERR_ALLOC;
+	}
+	t.halo = (int *)((char *)t.coef + csz);
+	t.bond = t.halo + (size_t)nh * tp;
+	EPHMC_HIP(hipMemcpy(t.halo, tab.data(), tsz, hipMemcpyHostToDevice));
+	return EPHMC_OK;
+}
+
+// Whether the chain of this arithmetic runs in the patch form: not with a shape set by
+// ephmc_autotune or by a tuning variable.
+bool patch_on(const ephmc_ctx *c, int prec)
+{
+	const int slot = prec == EPHMC_FP64 ? 0 : 1;
+	return c->patch[slot].cols && !c->chain_cols_set[slot] && c->chain_strip_set[slot] < 0 && !getenv("EPHMC_CHAIN_COLS")
+		&& !getenv("EPHMC_CHAIN_STRIP") && !getenv("EPHMC_CHAIN_SITES");
+}
+
+void patch_release(ephmc_ctx *c)
+{
+	for(PatchTab &t : c->patch){
+		if(t.coef) (void)hipFree(t.coef);
+		t = PatchTab{};
+	}
+}
+
 // Strip width for this lattice and arithmetic (0: site-per-thread form): the width chosen by
 // ephmc_autotune, else EPHMC_CHAIN_STRIP=0/2/4, else 2 in fp64 and 0 in fp32.  The strip form
 // cuts the LDS reads by a third (M = 2) at a larger register footprint; at 32x32 it is the
@@ -485,9 +766,36 @@ static ChainArgs<R> forward_args(ephmc_ctx *c, const R *coef, const void *src, v
 	return a;
 }
 
+// the patch form's coefficients are the current field's (coefficients() wrote them last) and in use
+static bool patch_ready(const ephmc_ctx *c, int prec)
+{
+	return c->patch_slot == (prec == EPHMC_FP64 ? 0 : 1) && patch_on(c, prec);
+}
+
+template <typename R>
+static int patch_chain(ephmc_ctx *c, const R *src, R *dst, R *ck, unsigned ck_every, int tau0, int dir, int ntau)
+{
+	const PatchTab &t = c->patch[sizeof(R) == 8 ? 0 : 1];
+	PatchArgs<R> a = patch_args<R>(c, t);
+	a.src = src;
+	a.dst = dst;
+	a.ck = ck;
+	a.ck_every = ck_every ? ck_every : 1;
+	a.tau0 = tau0;
+	a.dir = dir;
+	a.ntau = ntau;
+	return launch_patch<R>(c, t, a);
+}
+
 int chain_forward(ephmc_ctx *c, int prec, const void *src, void *dst, void *ck, unsigned ck_every,
 		int descending, bool from_identity)
 {
+	if(patch_ready(c, prec)){
+		const int tau0 = descending ? (int)c->nt - 1 : 0, dir = descending ? -1 : 1;
+		if(from_identity) src = nullptr;
+		if(prec == EPHMC_FP64) return patch_chain<double>(c, (const double *)src, (double *)dst, (double *)ck, ck_every, tau0, dir, (int)c->nt);
+		return patch_chain<float>(c, (const float *)src, (float *)dst, (float *)ck, ck_every, tau0, dir, (int)c->nt);
+	}
 	if(prec == EPHMC_FP64)
 		return launch_chain<double>(c, forward_args<double>(c, c->d_coef64, src, dst, ck, ck_every, descending, from_identity),
 			chain_cols(c, prec));
@@ -500,6 +808,7 @@ int chain_forward(ephmc_ctx *c, int prec, const void *src, void *dst, void *ck, 
 int chain_range(ephmc_ctx *c, int prec, const double *src, void *dst, int tau0, int dir, int ntau)
 {
 	if(prec == EPHMC_FP64){
+		if(patch_ready(c, prec)) return patch_chain<double>(c, src, (double *)dst, nullptr, 1, tau0, dir, ntau);
 		ChainArgs<double> a = make_args<double>(c, c->d_coef64);
 		a.src = src;
 		a.dst = (double *)dst;
@@ -513,6 +822,7 @@ int chain_range(ephmc_ctx *c, int prec, const double *src, void *dst, int tau0, 
 		s32 = (float *)c->d_seg;        // scratch: the segment buffer holds at least N^2 values
 		EPHMC_TRY(convert_f64_to_f32(c, src, s32, c->mat));
 	}
+	if(patch_ready(c, prec)) return patch_chain<float>(c, s32, (float *)dst, nullptr, 1, tau0, dir, ntau);
 	ChainArgs<float> a = make_args<float>(c, c->d_coef32);
 	a.src = s32;
 	a.dst = (float *)dst;

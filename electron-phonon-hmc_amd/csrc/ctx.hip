@@ -360,6 +360,7 @@ int ephmc_create(const ephmc_config *cfg, ephmc_ctx **out)
 	ephmc_ctx *c = new ephmc_ctx();
 	c->cfg = *cfg;
 	c->chain_strip_set[0] = c->chain_strip_set[1] = -1;
+	c->patch_slot = -1;
 	c->l1 = cfg->l1; c->l2 = cfg->l2; c->ns = ns; c->nt = cfg->nt; c->loc = 3 * ns;
 	c->dim = (size_t)c->nt * c->loc;
 	c->mat = (size_t)ns * ns;
@@ -448,6 +449,7 @@ int ephmc_create(const ephmc_config *cfg, ephmc_ctx **out)
 		set_error("initial uploads failed");
 		return fail(EPHMC_ERR_HIP);
 	}
+	if((rc = patch_reserve(c, EPHMC_FP64)) != EPHMC_OK || (mixed && (rc = patch_reserve(c, EPHMC_MIXED)) != EPHMC_OK)) return fail(rc);
 	// the stabilised product's buffers now, so that a captured trajectory allocates nothing
 	if(cfg->stabilize && (rc = stab_reserve(c)) != EPHMC_OK) return fail(rc);
 	if(cfg->schur_form_inv && (rc = schur_reserve(c)) != EPHMC_OK) return fail(rc);
@@ -464,6 +466,7 @@ int ephmc_destroy(ephmc_ctx *c)
 		c->d_Tfin32, c->d_gj[0], c->d_gj[1], c->d_piv, c->d_src, c->d_diag, c->d_dlu, c->d_scal, c->d_twiddle, c->d_f2, c->d_f2mom, c->d_red,
 		c->d_x, c->d_p, c->d_pdot, c->d_xnew, c->d_normals, c->d_minv, c->d_mhat, c->d_Rt0, c->d_R0t, c->d_ccg};
 	for(void *b : bufs) if(b) (void)hipFree(b);
+	patch_release(c);
 	tl_release(c);
 	stab_release(c);
 	schur_release(c);
@@ -946,6 +949,10 @@ int ephmc_autotune(ephmc_ctx *c, ephmc_tune_result *res)
 		const size_t csz = cprec == EPHMC_FP64 ? 8 : 4;
 		struct Shape { unsigned C, M; double ms; };
 		std::vector<Shape> shapes;
+		// C = 0: the patch form, where the context has it
+		c->chain_cols_set[slot] = 0;
+		c->chain_strip_set[slot] = -1;
+		if(patch_on(c, cprec)) shapes.push_back({0, 0, 1e30});
 		for(unsigned M : {0u, 2u, 4u}){
 			if(M && (c->l1 % M != 0 || ns / M > 1024)) continue;
 			for(unsigned C : {1u, 2u, 4u, 8u}){
@@ -958,7 +965,7 @@ int ephmc_autotune(ephmc_ctx *c, ephmc_tune_result *res)
 		for(int round = 0; round < 3; round++){
 			for(Shape &sh : shapes){
 				c->chain_cols_set[slot] = sh.C;
-				c->chain_strip_set[slot] = (int)sh.M;
+				c->chain_strip_set[slot] = sh.C ? (int)sh.M : -1;
 				double ms;
 				EPHMC_TRY(time_ms(c, e0, e1, 2, &ms, run));
 				if(ms < sh.ms) sh.ms = ms;
@@ -968,7 +975,11 @@ int ephmc_autotune(ephmc_ctx *c, ephmc_tune_result *res)
 		for(const Shape &sh : shapes)
 			if(sh.ms < ms_out){ ms_out = sh.ms; cols_out = sh.C; strip_out = sh.M; }
 		c->chain_cols_set[slot] = cols_out;
-		c->chain_strip_set[slot] = (int)strip_out;
+		c->chain_strip_set[slot] = cols_out ? (int)strip_out : -1;
+		if(cols_out == 0){
+			cols_out = c->patch[slot].cols;
+			strip_out = c->patch[slot].px == 2 && c->l1 % 2 == 0 ? 2 : 0;
+		}
 		return EPHMC_OK;
 	};
 	do {

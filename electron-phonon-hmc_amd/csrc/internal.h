@@ -100,6 +100,15 @@ struct StabWork {
 	int *perm = nullptr, *nref = nullptr;
 };
 
+// Tables of the patch form of the chain for one arithmetic (patch.h): columns per workgroup (0: not
+// used), sites per thread, patches per row, patches, places per LDS slot, bonds per patch; LDS
+// places of the halos, link of every bond, and the coefficients of the current field.
+struct PatchTab {
+	unsigned cols = 0, px = 0, py = 0, npx = 0, np = 0, tp = 0, nk = 0;
+	int *halo = nullptr, *bond = nullptr;
+	void *coef = nullptr;
+};
+
 } // namespace ephmc
 
 struct ephmc_ctx {
@@ -119,6 +128,8 @@ struct ephmc_ctx {
 	// slice coefficients
 	double *d_coef64;                 // [nt][6][ns]
 	float *d_coef32;
+	ephmc::PatchTab patch[2];         // [0] fp64, [1] fp32
+	int patch_slot;                   // the one whose coefficients are the current field's, or -1
 
 	// chain / force workspace
 	unsigned ckpt;                    // k: T stored every k slices (k = 1: every slice, read back directly)
@@ -241,6 +252,9 @@ int timer_end(ephmc_ctx *c, const char *group);
 // chain.hip
 unsigned sites_per_thread(const char *var);
 unsigned strip_width(const ephmc_ctx *c, int prec);
+int patch_reserve(ephmc_ctx *c, int prec);
+bool patch_on(const ephmc_ctx *c, int prec);
+void patch_release(ephmc_ctx *c);
 int coefficients(ephmc_ctx *c, const double *x, bool want32);
 int chain_forward(ephmc_ctx *c, int prec, const void *src, void *dst, void *ck, unsigned ck_every,
 		int descending, bool from_identity);

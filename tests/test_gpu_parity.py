@@ -62,6 +62,24 @@ def test_strip_chain_bit_identical(monkeypatch, l1, l2, nt, strip):
     np.testing.assert_array_equal(Ms, Mg)
 
 
+# every shape of the patch form (one site up to 512 / 640 sites, 2 x 2 sites beyond, more than 512
+# threads), extents that are no multiple of the patch, lattices of one row or column, orders 2 and 6
+@pytest.mark.parametrize("l1,l2,nt,order", [(1, 1, 2, 4), (5, 4, 3, 4), (1, 40, 3, 4), (64, 1, 3, 2), (16, 16, 3, 6), (21, 19, 3, 4),
+                                            (25, 25, 3, 4), (27, 31, 3, 4), (32, 32, 3, 6), (33, 32, 2, 4), (700, 1, 2, 4),
+                                            (1, 1001, 2, 4), (45, 45, 2, 4), (64, 32, 2, 2)])
+def test_patch_chain_bit_identical(monkeypatch, l1, l2, nt, order):
+    """The patch form of the chain sums in the order of the site form: M_hat (fp64) and the mixed
+    molecular-dynamics force (fp32 chain) agree to the last bit (EPHMC_CHAIN_STRIP=0: the site form)."""
+    say("patch vs site chain", l1, l2, nt, order)
+    om = OracleModel(l1, l2, nt, beta=nt * 40 / 32, taylor=order)
+    ctx = gpu_context(om, precision=1, taylor_order=order)
+    x = field(om, 5)
+    Mp, Fp = ctx.M_hat(x), ctx.md_force(x)
+    monkeypatch.setenv("EPHMC_CHAIN_STRIP", "0")
+    np.testing.assert_array_equal(Mp, ctx.M_hat(x))
+    np.testing.assert_array_equal(Fp, ctx.md_force(x))
+
+
 @pytest.mark.parametrize("revert,stop", [(0, 2), (0, 1), (0, 0), (1, 0), (1, -1)])
 def test_apply_exp_partial(revert, stop):
     say("apply_exp_M", revert, stop)
