@@ -74,9 +74,12 @@ struct TlWork {
 	unsigned cap_b = 0, cap_nbins = 0;
 	size_t rot_cap = 0;               // rotations recorded per sample
 	unsigned sw_cap = 0;              // sweeps recorded per sample
-	double *A = nullptr, *Z = nullptr;   // [B][N][N]; the sorted eigenvectors V reuse A
+	double *A = nullptr, *Z = nullptr;   // [B][N][N]; the eigenvectors, unsorted and sorted, reuse both
 	double2 *rot = nullptr;           // [B][rot_cap] (c, s); W_0, W_1 ([B][N][N] each) reuse it
-	double *V = nullptr, *W0 = nullptr, *W1 = nullptr;
+	double *W0 = nullptr, *W1 = nullptr;
+	double4 *ts = nullptr;            // [B][N] scaled tridiagonal matrix; tn[B] its scale
+	double *tn = nullptr, *rn = nullptr;   // rn: 1 / |vector|
+	int *ql = nullptr;                // [B] sample takes the QL iteration
 	int4 *sw = nullptr;               // [B][sw_cap] (first rotation, lowest, highest position)
 	unsigned *nsw = nullptr;
 	int *status = nullptr, *perm = nullptr;

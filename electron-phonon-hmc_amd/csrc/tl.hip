@@ -19,6 +19,11 @@
 //                   rank-2 update of step j fused with the matrix-vector product of step j+1
 //                   (read and written once per step).  Reflectors v_j overwrite column j below
 //                   the diagonal.
+//   tl_bisect       (3 <= N <= 1024) eigenvalues by bisection with Sturm counts, one per thread
+//   tl_vectors      eigenvectors of the tridiagonal matrix by twisted factorisation, one per thread;
+//                   tl_orthogonalise makes neighbours with a small gap orthogonal.  A sample where
+//                   that does not hold (eigenvalues equal to rounding) takes the QL iteration below,
+//                   as all samples of the other sizes do:
 //   tl_ql_scalar    implicit QL with Wilkinson shifts on (d, e) (the scalar recurrence of the
 //                   EISPACK tql2 method, one wave per sample computing it in every lane),
 //                   recording every rotation (c, s) and the position range of every sweep
@@ -77,6 +82,16 @@ __device__ double block_sum(double v, double *red)
 	for(int q = 0; q < BT / 64; q++) t += red[q];
 	__syncthreads();
 	return t;
+}
+
+// 1/x: hardware reciprocal refined by two Newton steps
+__device__ inline double rcp_nr(double x)
+{
+	double r = __builtin_amdgcn_rcp(x);
+	double t = fma(-x, r, 1.0);
+	r = fma(r, t, r);
+	t = fma(-x, r, 1.0);
+	return fma(r, t, r);
 }
 
 // ---- H ----------------------------------------------------------------------------------
@@ -560,22 +575,232 @@ __global__ __launch_bounds__(BT) void tl_tridiag_panel_kernel(double *__restrict
 	}
 }
 
+// ---- eigenvalues and eigenvectors of the tridiagonal matrix, one per thread ------------------
+// The QL iteration below is one chain of about 0.9 N^2 rotations per sample, 265 ns each, whose vector part
+// repeats 6 flops N times per rotation: 330 of the 506 ms of 256 samples at N = 1024.  Here every
+// eigenvalue and every vector is its own chain of N steps (bisection: N steps per bit), N of them side
+// by side on a CU: 4 ms for both.
+//
+// ts[s][i] = (d_i, e_{i-1}^2, e_i, 0) scaled by 1 / B, B >= every |eigenvalue| a power of two, so the
+// scaling is exact; e^2 at least 2^-112 (a change of e by 2^-56 of the norm), so that the Sturm
+// sequence cannot underflow between its rescalings.  Read through the scalar cache: every lane
+// wants the same entry.
+__global__ __launch_bounds__(256) void tl_scale_kernel(const double *__restrict__ dall, const double *__restrict__ eall, unsigned n,
+		double4 *__restrict__ tsall, double *__restrict__ tn, int *__restrict__ ql, int *__restrict__ status)
+{
+	__shared__ double red[4];
+	const unsigned s = blockIdx.x, tid = threadIdx.x;
+	const double *d = dall + (size_t)s * n, *e = eall + (size_t)s * n;
+	double m = 0;
+	bool bad = false;
+	for(unsigned i = tid; i < n; i += 256){
+		const double r = fabs(d[i]) + (i ? fabs(e[i - 1]) : 0.0) + (i + 1 < n ? fabs(e[i]) : 0.0);
+		bad |= !(r < HUGE_VAL);
+		m = fmax(m, r);
+	}
+#pragma unroll
+	for(int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+	if((tid & 63) == 0) red[tid >> 6] = m;
+	const int anybad = __syncthreads_or(bad);
+	m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+	// 2^k >= m; a zero matrix keeps scale 1, NaN or infinity goes to the QL iteration
+	const int k = m > 0 && !anybad ? __builtin_amdgcn_frexp_exp(m) : 0;
+	const double sc = ldexp(1.0, -k);
+	for(unsigned i = tid; i < n; i += 256){
+		const double el = i ? e[i - 1] * sc : 0.0;
+		tsall[(size_t)s * n + i] = make_double4(d[i] * sc, i ? fmax(el * el, 0x1p-112) : 0.0, i + 1 < n ? e[i] * sc : 0.0, 0.0);
+	}
+	if(tid == 0){
+		tn[s] = ldexp(1.0, k);
+		ql[s] = anybad;
+		status[s] = 0;
+	}
+}
+
+// Number of eigenvalues below x: sign changes of p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2}, no division;
+// both terms rescaled every 8 steps (a step grows at most by 3, shrinks at least by 2^-112)
+__device__ __forceinline__ unsigned tl_count(const double4 *__restrict__ ts, unsigned n, double x)
+{
+	double p0 = 1.0, p1 = ts[0].x - x;
+	unsigned cnt = (unsigned)(__double_as_longlong(p1) < 0);
+	unsigned i = 1;
+	for(; i + 8 <= n; i += 8){
+#pragma unroll
+		for(int u = 0; u < 8; u++){
+			const double p2 = fma(ts[i + u].x - x, p1, -(ts[i + u].y * p0));
+			cnt += (unsigned)(__double2hiint(p2) ^ __double2hiint(p1)) >> 31;
+			p0 = p1;
+			p1 = p2;
+		}
+		const int k = -__builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(p1)));
+		p0 = ldexp(p0, k);
+		p1 = ldexp(p1, k);
+	}
+	for(; i < n; i++){
+		const double p2 = fma(ts[i].x - x, p1, -(ts[i].y * p0));
+		cnt += (unsigned)(__double2hiint(p2) ^ __double2hiint(p1)) >> 31;
+		p0 = p1;
+		p1 = p2;
+	}
+	return cnt;
+}
+
+// Eigenvalue k (ascending) on thread k of the sample's workgroup (blockDim.x >= n): one round of counts on
+// a grid of blockDim.x points shared by all threads, then bisection to 2^-53 of the norm.
+__global__ __launch_bounds__(1024) void tl_bisect_kernel(const double4 *__restrict__ tsall, const double *__restrict__ tn, unsigned n,
+		double *__restrict__ evall)
+{
+	__shared__ unsigned grid[1024];
+	const unsigned s = blockIdx.x, k = threadIdx.x, bt = blockDim.x;
+	const double4 *ts = tsall + (size_t)s * n;
+	const double h = 2.0 / bt;
+	grid[k] = tl_count(ts, n, -1.0 + h * k);
+	__syncthreads();
+	// the last grid point with at most k eigenvalues below it
+	unsigned a = 0, b = bt;
+	while(b - a > 1){
+		const unsigned m = (a + b) / 2;
+		if(grid[m] <= k) a = m;
+		else b = m;
+	}
+	if(k >= n) return;
+	double lo = -1.0 + h * a, hi = lo + h;
+	for(int it = 0; it < 60 && hi - lo > 0x1p-54; it++){
+		const double x = 0.5 * (lo + hi);
+		if(x <= lo || x >= hi) break;
+		if(tl_count(ts, n, x) > k) hi = x;
+		else lo = x;
+	}
+	evall[(size_t)s * n + k] = 0.5 * (lo + hi) * tn[s];
+}
+
+// Eigenvector k of the scaled tridiagonal matrix for eigenvalue ev[k] by twisted factorisation, thread = k.
+// D+ (from the top) and D- (from the bottom) are the pivots of T - x; with
+//     l_i = e_i / D+_i,  u_i = e_i / D-_{i+1},  gamma_i = d_i - x - l_{i-1} e_{i-1} - u_i e_i,
+// the vector with z_r = 1, z_i = -l_i z_{i+1} above and z_{i+1} = -u_i z_i below satisfies every row of
+// T - x but row r, which leaves gamma_r: r is where |gamma| is smallest.  Each relation is local, so
+// rounding leaves a residual of eps |T| in every row whatever the pivots' size; a pivot below
+// 2^-52 is moved there, a change of d by as much.  l, u and z: [i][k], lanes on consecutive k.
+// rn = 1 / |z|.  A residual above 1e-13 sends the sample to the QL iteration.
+__global__ __launch_bounds__(256) void tl_vectors_kernel(const double4 *__restrict__ tsall, const double *__restrict__ tn,
+		const double *__restrict__ evall, unsigned n, double *__restrict__ lu, size_t lu_stride, double *__restrict__ Zall,
+		double *__restrict__ rnall, int *__restrict__ ql)
+{
+	const unsigned s = blockIdx.y, k = blockIdx.x * 256 + threadIdx.x;
+	if(k >= n || ql[s]) return;
+	const double4 *ts = tsall + (size_t)s * n;
+	double *L = lu + (size_t)s * lu_stride + k, *U = L + (size_t)n * n, *Z = Zall + (size_t)s * n * n + k;
+	const double x = evall[(size_t)s * n + k] / tn[s];
+	auto pivot = [](double d){ return fabs(d) < 0x1p-52 ? copysign(0x1p-52, d) : d; };
+	double le = 0;                                   // l_{i-1} e_{i-1}
+#pragma unroll 4
+	for(unsigned i = 0; i + 1 < n; i++){
+		const double e = ts[i].z, l = e * rcp_nr(pivot(ts[i].x - x - le));
+		L[(size_t)i * n] = l;
+		le = l * e;
+	}
+	double best = HUGE_VAL, ue = 0;                  // u_i e_i
+	unsigned r = 0;
+#pragma unroll 4
+	for(unsigned i = n - 1; i > 0; i--){
+		const double e = ts[i - 1].z, dx = ts[i].x - x, dm = dx - ue;       // D-_i
+		const double g = fabs(dm - L[(size_t)(i - 1) * n] * e), u = e * rcp_nr(pivot(dm));
+		if(g < best){ best = g; r = i; }
+		U[(size_t)(i - 1) * n] = u;
+		ue = u * e;
+	}
+	{
+		const double g = fabs(ts[0].x - x - ue);
+		if(g < best){ best = g; r = 0; }
+	}
+	double ss = 1.0, z = 1.0;
+	Z[(size_t)r * n] = 1.0;
+#pragma unroll 4
+	for(unsigned i = n - 1; i > 0; i--){
+		const double l = L[(size_t)(i - 1) * n];
+		if(i <= r){
+			z *= -l;
+			Z[(size_t)(i - 1) * n] = z;
+			ss = fma(z, z, ss);
+		}
+	}
+	z = 1.0;
+#pragma unroll 4
+	for(unsigned i = 0; i + 1 < n; i++){
+		const double u = U[(size_t)i * n];
+		if(i >= r){
+			z *= -u;
+			Z[(size_t)(i + 1) * n] = z;
+			ss = fma(z, z, ss);
+		}
+	}
+	const double rn = 1.0 / sqrt(ss);
+	rnall[(size_t)s * n + k] = rn;
+	if(!(best * rn < 1e-13)) ql[s] = 1;
+}
+
+// Vectors whose eigenvalues differ by less than 2^-14 of the norm, made orthogonal one after the other
+// within each run of such neighbours (beyond it eps / gap bounds the overlap by 4e-12).  Of a run's
+// space any orthonormal basis serves: the pairs it forms share their bins to 2^-14 of the norm and
+// their weights' sum does not depend on the basis.  Vectors that nearly coincide (overlap above 0.85),
+// or a run of more than 16, send the sample to the QL iteration.
+__global__ __launch_bounds__(256) void tl_orthogonalise_kernel(const double *__restrict__ evall, const double *__restrict__ tn, unsigned n,
+		double *__restrict__ Zall, double *__restrict__ rnall, int *__restrict__ ql)
+{
+	__shared__ double red[4];
+	__shared__ unsigned char near_[1024];
+	const unsigned s = blockIdx.x, tid = threadIdx.x;
+	if(ql[s]) return;
+	const double *ev = evall + (size_t)s * n;
+	const double tol = 0x1p-14 * tn[s];
+	int any = 0;
+	for(unsigned k = tid; k < n; k += 256){
+		const int c = k > 0 && ev[k] - ev[k - 1] < tol;
+		near_[k] = (unsigned char)c;
+		any |= c;
+	}
+	if(!__syncthreads_or(any)) return;
+	double *Z = Zall + (size_t)s * n * n, *rn = rnall + (size_t)s * n;
+	unsigned first = 0;
+	for(unsigned k = 1; k < n; k++){
+		if(!near_[k]){
+			first = k;
+			continue;
+		}
+		if(k - first > 16){
+			if(tid == 0) ql[s] = 1;
+			return;
+		}
+		// z_k (normalised) minus its projections on the run's vectors so far
+		double left = 1.0;
+		for(unsigned q = first; q < k; q++){
+			double t = 0;
+			for(unsigned i = tid; i < n; i += 256) t = fma(Z[(size_t)i * n + q], Z[(size_t)i * n + k], t);
+			t = block_sum<256>(t, red);
+			const double rq = rn[q], c = t * rq * rq;        // z_k -= (z_q . z_k / |z_q|^2) z_q
+			left -= t * t * rq * rq * rn[k] * rn[k];
+			for(unsigned i = tid; i < n; i += 256) Z[(size_t)i * n + k] = fma(-c, Z[(size_t)i * n + q], Z[(size_t)i * n + k]);
+			__syncthreads();
+		}
+		if(!(left > 0.28)){
+			if(tid == 0) ql[s] = 1;
+			return;
+		}
+		double t = 0;
+		for(unsigned i = tid; i < n; i += 256) t = fma(Z[(size_t)i * n + k], Z[(size_t)i * n + k], t);
+		t = block_sum<256>(t, red);
+		__syncthreads();
+		if(tid == 0) rn[k] = 1.0 / sqrt(t);
+		__syncthreads();
+	}
+}
+
 // ---- implicit QL: scalar recurrence ----------------------------------------------------------
 // e[i] couples i and i+1.  Rotation (c, s) at position i acts on columns (i, i+1) of Z:
 // Z(:,i+1) <- s Z(:,i) + c Z(:,i+1),  Z(:,i) <- c Z(:,i) - s Z(:,i+1).  Sweep records: (first
 // rotation index, lowest position, highest position); positions run from high to low.
 // One wave per sample runs the recurrence with every lane computing the same values (d, e in
 // LDS, written by all lanes alike); the deflation test scans 64 positions per step.
-
-// 1/x: hardware reciprocal refined by two Newton steps
-__device__ inline double rcp_nr(double x)
-{
-	double r = __builtin_amdgcn_rcp(x);
-	double t = fma(-x, r, 1.0);
-	r = fma(r, t, r);
-	t = fma(-x, r, 1.0);
-	return fma(r, t, r);
-}
 
 // sqrt(f^2 + g^2): the plain form while the square sum is a normal number, hypot otherwise
 __device__ inline double norm2(double f, double g)
@@ -587,11 +812,12 @@ __device__ inline double norm2(double f, double g)
 
 __global__ __launch_bounds__(64) void tl_ql_scalar_kernel(const double *__restrict__ dall, const double *__restrict__ eall,
 		unsigned n, double *__restrict__ evall, double2 *__restrict__ rotall, size_t rot_cap, int4 *__restrict__ swall,
-		unsigned sw_cap, unsigned *__restrict__ nsw_all, int *__restrict__ status)
+		unsigned sw_cap, unsigned *__restrict__ nsw_all, int *__restrict__ status, const int *__restrict__ ql)
 {
 	extern __shared__ double sh[];
 	double *d = sh, *e = sh + n;
 	const unsigned s = blockIdx.x, lane = threadIdx.x;
+	if(ql && !ql[s]) return;
 	for(unsigned i = lane; i < n; i += 64){
 		d[i] = dall[(size_t)s * n + i];
 		e[i] = i + 1 < n ? eall[(size_t)s * n + i] : 0.0;
@@ -732,12 +958,14 @@ __device__ __forceinline__ bool tl_ql_turn(double (&R)[G + 1 + PF], const double
 
 template <int G, int PF, int QC>
 __global__ __launch_bounds__(256) void tl_ql_apply_kernel(double *__restrict__ Zall, unsigned n, const double2 *__restrict__ rotall,
-		size_t rot_cap, const int4 *__restrict__ swall, unsigned sw_cap, const unsigned *__restrict__ nsw_all)
+		size_t rot_cap, const int4 *__restrict__ swall, unsigned sw_cap, const unsigned *__restrict__ nsw_all,
+		const int *__restrict__ ql)
 {
 	constexpr int NR = G + 1 + PF;
 	static_assert(QC % NR == 0, "a stage is whole turns of the ring");
 	__shared__ double2 rs[QC][G];
 	const unsigned s = blockIdx.y;
+	if(ql && !ql[s]) return;
 	const unsigned r = blockIdx.x * 256 + threadIdx.x;
 	const bool act = r < n;
 	double *Z = Zall + (size_t)s * n * n;
@@ -937,9 +1165,12 @@ __global__ __launch_bounds__(256) void tl_wy_t_kernel(const double *__restrict__
 // l, element e = row 4 e + l / 16, column l % 16) for the whole sweep over the blocks, so Z is read
 // and written once.  Per block: W^T = Z^T Y (each wave over its rows; the accumulator elements
 // serve directly as the A operand, rows 16 q + 4 e + l / 16 of step (q, e)), the eight waves'
-// parts summed in LDS, W2^T = W^T T^T, then Z -= Y W2 (v_mfma_f64_16x16x4 both ways).
+// parts summed in LDS, W2^T = W^T T^T, then Z -= Y W2 (v_mfma_f64_16x16x4 both ways).  Z comes as [row][column]
+// with 1 / |column| in rn from the twisted factorisations, or by columns from the QL iteration (ql[s]);
+// V is written by columns.
 __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *__restrict__ Yball, const double *__restrict__ Tall,
-		unsigned n, unsigned nblk, double *__restrict__ Zall)
+		unsigned n, unsigned nblk, const double *__restrict__ Zall, const double *__restrict__ rnall, const int *__restrict__ ql,
+		double *__restrict__ Vall)
 {
 	typedef double v4d __attribute__((ext_vector_type(4)));
 	__shared__ double Ts[TL_WB][TL_WB + 1];
@@ -949,16 +1180,19 @@ __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *_
 	const unsigned s = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 	const unsigned g = lane >> 4, m = lane & 15, c0 = blockIdx.x * TL_WC, n16 = (n + 15) & ~15u;
 	const double *Tb = Tall + (size_t)s * nblk * TL_WB * TL_WB;
-	double *Z = Zall + (size_t)s * n * n;
+	const double *Z = Zall + (size_t)s * n * n;
+	double *V = Vall + (size_t)s * n * n;
 	const unsigned rw0 = wave * 16 * TL_WRB;                      // first row of this wave
 	const unsigned col = c0 + m;
+	const bool by_col = ql[s] != 0;
+	const double rn = by_col || col >= n ? 1.0 : rnall[(size_t)s * n + col];
 	v4d acc[TL_WRB];
 #pragma unroll
 	for(int q = 0; q < TL_WRB; q++)
 #pragma unroll
 		for(int e = 0; e < 4; e++){
 			const unsigned r = rw0 + 16 * q + 4 * e + g;
-			acc[q][e] = (r < n && col < n) ? Z[(size_t)col * n + r] : 0.0;
+			acc[q][e] = (r < n && col < n) ? rn * Z[by_col ? (size_t)col * n + r : (size_t)r * n + col] : 0.0;
 		}
 	for(int b = (int)nblk - 1; b >= 0; b--){
 		const unsigned jb = (unsigned)b * TL_WB;
@@ -1024,7 +1258,7 @@ __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *_
 #pragma unroll
 		for(int e = 0; e < 4; e++){
 			const unsigned r = rw0 + 16 * q + 4 * e + g;
-			if(r < n && col < n) Z[(size_t)col * n + r] = acc[q][e];
+			if(r < n && col < n) V[(size_t)col * n + r] = acc[q][e];
 		}
 }
 
@@ -1338,14 +1572,14 @@ static int tl_reserve(ephmc_ctx *c, unsigned B, unsigned nbins)
 		|| (rc = al((void **)&w.ev, B * (size_t)n * 8)) || (rc = al((void **)&w.evs, B * (size_t)n * 8))
 		|| (rc = al((void **)&w.ems, B * (size_t)n * 8)) || (rc = al((void **)&w.perm, B * (size_t)n * sizeof(int)))
 		|| (rc = al((void **)&w.res, B * 8)) || (rc = al((void **)&w.part, B * (size_t)nblk * nblk * nbins * 8))
+		|| (rc = al((void **)&w.ts, B * (size_t)n * sizeof(double4))) || (rc = al((void **)&w.tn, B * 8))
+		|| (rc = al((void **)&w.rn, B * (size_t)n * 8)) || (rc = al((void **)&w.ql, B * sizeof(int)))
 		|| (rc = al((void **)&w.acc, (size_t)nbins * 8))
 		|| (rc = al((void **)&w.red, ((B * (size_t)nblk * nblk + TL_RC - 1) / TL_RC) * nbins * 8))){
 		tl_release(c);
 		return rc;
 	}
-	// A is free once the back-transformation has run, the rotations once they are applied
-	// (2 N^2 doubles fit in 1.5 N^2 double pairs)
-	w.V = w.A;
+	// the rotations are free once they are applied (2 N^2 doubles fit in 1.5 N^2 double pairs)
 	w.W0 = (double *)w.rot;
 	w.W1 = (double *)w.rot + B * mat;
 	w.cap_b = B;
@@ -1357,7 +1591,7 @@ void tl_release(ephmc_ctx *c)
 {
 	TlWork &w = c->tl;
 	void *bufs[] = {w.A, w.Z, w.rot, w.red, w.sw, w.nsw, w.status, w.x, w.d, w.e, w.tau, w.ev, w.evs, w.ems, w.perm,
-		w.res, w.part, w.acc};
+		w.res, w.part, w.acc, w.ts, w.tn, w.rn, w.ql};
 	for(void *b : bufs) if(b) (void)hipFree(b);
 	w = TlWork();
 }
@@ -1416,40 +1650,56 @@ extern "C" int ephmc_tl_hist(ephmc_ctx *c, const double *normals, unsigned nsamp
 			EPHMC_LAUNCHED();
 		}
 		EPHMC_TRY(timer_end(c, "tl_tridiag"));
+		// back-transformation in compact-WY blocks on the matrix cores (N <= 1024), the reflector copy and
+		// the T factors in the rotation buffer, which is free by then; else one reflector at a time
+		const unsigned nblkw = n > 2 ? (n - 2 + TL_WB - 1) / TL_WB : 0;
+		const size_t ybsz = (size_t)nblkw * ((n + 15) & ~15u) * TL_WB;
+		const bool wy = n >= 3 && n <= TL_WW * 16 * TL_WRB && ybsz + (size_t)nblkw * TL_WB * TL_WB <= 2 * w.rot_cap;
 		EPHMC_TRY(timer_begin(c, "tl_ql"));
+		if(wy){
+			// one thread per eigenvalue and per vector; the samples that need the QL iteration are marked
+			tl_scale_kernel<<<nb_, 256, 0, c->stream>>>(w.d, w.e, n, w.ts, w.tn, w.ql, w.status);
+			EPHMC_LAUNCHED();
+			tl_bisect_kernel<<<nb_, (n + 63) & ~63u, 0, c->stream>>>(w.ts, w.tn, n, w.ev);
+			EPHMC_LAUNCHED();
+			tl_vectors_kernel<<<dim3((n + 255) / 256, nb_), 256, 0, c->stream>>>(w.ts, w.tn, w.ev, n, (double *)(void *)w.rot, 2 * w.rot_cap,
+				w.Z, w.rn, w.ql);
+			EPHMC_LAUNCHED();
+			tl_orthogonalise_kernel<<<nb_, 256, 0, c->stream>>>(w.ev, w.tn, n, w.Z, w.rn, w.ql);
+			EPHMC_LAUNCHED();
+		}
+		const int *ql = wy ? w.ql : nullptr;
 		tl_ql_scalar_kernel<<<nb_, 64, 2 * (size_t)n * 8, c->stream>>>(w.d, w.e, n, w.ev, w.rot, w.rot_cap, w.sw, w.sw_cap, w.nsw,
-			w.status);
+			w.status, ql);
 		EPHMC_LAUNCHED();
-		tl_ql_apply_kernel<TL_G, TL_PF, TL_QC><<<dim3((n + 255) / 256, nb_), 256, 0, c->stream>>>(w.Z, n, w.rot, w.rot_cap, w.sw, w.sw_cap, w.nsw);
+		tl_ql_apply_kernel<TL_G, TL_PF, TL_QC><<<dim3((n + 255) / 256, nb_), 256, 0, c->stream>>>(w.Z, n, w.rot, w.rot_cap, w.sw, w.sw_cap,
+			w.nsw, ql);
 		EPHMC_LAUNCHED();
 		EPHMC_TRY(timer_end(c, "tl_ql"));
 		EPHMC_TRY(timer_begin(c, "tl_back"));
-		{
-			// compact-WY blocks on the matrix cores (N <= 1024), the reflector copy and the T factors in
-			// the rotation buffer, which is free once the rotations are applied; else one reflector at a time
-			const unsigned nblkw = n > 2 ? (n - 2 + TL_WB - 1) / TL_WB : 0;
-			const size_t ybsz = (size_t)nblkw * ((n + 15) & ~15u) * TL_WB;
+		const double *vec = w.Z;          // eigenvectors by columns, in the order of w.ev
+		if(wy){
 			double *yball = (double *)(void *)w.rot, *tall = yball + (size_t)nb_ * ybsz;
-			const bool wy = n >= 3 && n <= TL_WW * 16 * TL_WRB && ybsz + (size_t)nblkw * TL_WB * TL_WB <= 2 * w.rot_cap;
-			if(wy){
-				tl_yb_kernel<<<dim3((n + 31) / 32, nblkw, nb_), 256, 0, c->stream>>>(w.A, n, nblkw, yball);
-				EPHMC_LAUNCHED();
-				tl_wy_t_kernel<<<dim3(nblkw, nb_), 256, 0, c->stream>>>(w.A, w.tau, n, tall);
-				EPHMC_LAUNCHED();
-				tl_wy_apply_kernel<<<dim3((n + TL_WC - 1) / TL_WC, nb_), 64 * TL_WW, 0, c->stream>>>(yball, tall, n, nblkw, w.Z);
-			}else if(n <= 1024) tl_back_kernel<16, 4><<<dim3((n + 15) / 16, nb_), 256, 0, c->stream>>>(w.A, w.tau, w.Z, n);
-			else tl_back_kernel<32, 2><<<dim3((n + 7) / 8, nb_), 256, 0, c->stream>>>(w.A, w.tau, w.Z, n);
+			tl_yb_kernel<<<dim3((n + 31) / 32, nblkw, nb_), 256, 0, c->stream>>>(w.A, n, nblkw, yball);
 			EPHMC_LAUNCHED();
-		}
+			tl_wy_t_kernel<<<dim3(nblkw, nb_), 256, 0, c->stream>>>(w.A, w.tau, n, tall);
+			EPHMC_LAUNCHED();
+			// (the reflectors' copy is made: A takes the vectors)
+			tl_wy_apply_kernel<<<dim3((n + TL_WC - 1) / TL_WC, nb_), 64 * TL_WW, 0, c->stream>>>(yball, tall, n, nblkw, w.Z, w.rn, w.ql, w.A);
+			vec = w.A;
+		}else if(n <= 1024) tl_back_kernel<16, 4><<<dim3((n + 15) / 16, nb_), 256, 0, c->stream>>>(w.A, w.tau, w.Z, n);
+		else tl_back_kernel<32, 2><<<dim3((n + 7) / 8, nb_), 256, 0, c->stream>>>(w.A, w.tau, w.Z, n);
+		EPHMC_LAUNCHED();
+		double *sorted = vec == w.A ? w.Z : w.A;
 		EPHMC_TRY(timer_end(c, "tl_back"));
 		tl_sort_kernel<TL_BT><<<nb_, TL_BT, ((size_t)n + TL_BT / 64) * 8, c->stream>>>(w.ev, n, w.evs, w.ems, w.perm, w.res);
 		EPHMC_LAUNCHED();
-		tl_current_kernel<<<dim3(n, nb_), 256, (size_t)n * 8, c->stream>>>(w.Z, w.perm, w.x, c->d_nb, n, c->cfg.t[0], c->cfg.t[1],
+		tl_current_kernel<<<dim3(n, nb_), 256, (size_t)n * 8, c->stream>>>(vec, w.perm, w.x, c->d_nb, n, c->cfg.t[0], c->cfg.t[1],
 			c->cfg.t[2], c->cfg.kappa[0], c->cfg.kappa[1], c->cfg.kappa[2], contr_mat[0], contr_mat[1], contr_mat[2],
-			contr_mat[3], contr_mat[4], contr_mat[5], w.V, w.W0, w.W1);
+			contr_mat[3], contr_mat[4], contr_mat[5], sorted, w.W0, w.W1);
 		EPHMC_LAUNCHED();
 		EPHMC_TRY(timer_begin(c, "tl_pairs"));
-		tl_pairs_kernel<<<dim3(nblk, nblk, nb_), 256, 0, c->stream>>>(w.V, w.W0, w.W1, w.evs, w.ems, n, width, nbins, w.part);
+		tl_pairs_kernel<<<dim3(nblk, nblk, nb_), 256, 0, c->stream>>>(sorted, w.W0, w.W1, w.evs, w.ems, n, width, nbins, w.part);
 		EPHMC_LAUNCHED();
 		{
 			const unsigned nparts = nb_ * nblk * nblk, nch = (nparts + TL_RC - 1) / TL_RC;

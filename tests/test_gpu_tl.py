@@ -137,3 +137,27 @@ def test_tl_repeatable_and_additive():
     gb, zb = ctx.tl_hist(xs[7:], CM, width, nbins)
     np.testing.assert_array_equal(np.concatenate([za, zb]), z1)
     assert rel(ga + gb, g1) < 1e-14
+
+
+# Disorder that varies along one lattice direction only leaves the momentum of the other, and levels
+# of opposite momenta are degenerate in pairs; a random part of the given size splits them: from
+# equal to rounding (the QL iteration) over close pairs that are made orthogonal to separate levels.
+# N at the edges of a wave and of a workgroup.
+@pytest.mark.parametrize("l1,l2", [(3, 3), (6, 6), (8, 8), (13, 5), (16, 16), (19, 27)])
+@pytest.mark.parametrize("scale", [0.0, 1e-13, 1e-9, 1e-6, 1e-4, 1e-2])
+def test_tl_degenerate_pairs(l1, l2, scale):
+    """Bins above the first against LAPACK (the first holds the pairs inside a doublet, which count once
+    or twice as rounding orders their levels); the others do not depend on the basis chosen inside a
+    doublet.  Tolerances of this file."""
+    nbins = 96
+    om, width = tl_model(l1, l2, nbins)
+    rng = np.random.default_rng(31)
+    base = np.tile(rng.standard_normal((2, 1, l1, 3)), (1, l2, 1, 1)).reshape(2, -1)
+    xs = base + scale * rng.standard_normal(base.shape)
+    say("degenerate TL", l1, l2, scale)
+    ctx = gpu_context(om)
+    g, z = ctx.tl_hist(xs, CM, width, nbins)
+    ref = [numpy_tl(om, x, width, nbins) for x in xs]
+    gr, zr = sum(r[0] for r in ref), np.array([r[1] for r in ref])
+    assert np.abs(z / zr - 1).max() < 1e-12
+    assert rel(g[1:], gr[1:]) < 1e-9
