@@ -63,6 +63,22 @@ constexpr int TL_KC = 16;       // rows of V / W per LDS stage of the pair tiles
 constexpr unsigned TL_HB = 512; // bins a pair tile accumulates in LDS (wider tiles bin by search)
 constexpr unsigned TL_NONE = 0xffffffffu;
 
+// Sample and work item of workgroup b of a grid of `per` items for each of ns samples.  Workgroups go
+// to the eight XCDs in turn, so eight samples at a time run one to an XCD, whose L2 then holds
+// what the sample's workgroups share; samples past the last multiple of eight come one after the other.
+__device__ __forceinline__ void tl_item(unsigned b, unsigned per, unsigned ns, unsigned &s, unsigned &item)
+{
+	const unsigned full = ns / 8 * 8;
+	if(b < full * per){
+		s = b / (8 * per) * 8 + b % 8;
+		item = b / 8 % per;
+	}else{
+		const unsigned r = b - full * per;
+		s = full + r / per;
+		item = r % per;
+	}
+}
+
 __device__ inline double wave_sum(double v)
 {
 #pragma unroll
@@ -128,8 +144,16 @@ __device__ double tl_reflector(double *A, unsigned n, unsigned j, double *vb, do
 		const unsigned r = threadIdx.x + q * BT;
 		if(r >= j + 2 && r < n) ss += vb[r] * vb[r];
 	}
-	ss = block_sum<BT>(ss, red);
+	// block_sum, with alpha read between its barriers: vb is complete at the first, and the thread of row
+	// j + 1 overwrites its entry after the second
+	ss = wave_sum(ss);
+	if((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+	__syncthreads();
 	const double alpha = vb[j + 1];
+	ss = 0;
+#pragma unroll
+	for(int q = 0; q < BT / 64; q++) ss += red[q];
+	__syncthreads();
 	double tj = 0, beta = alpha, scale = 0;
 	if(ss != 0){
 		beta = -copysign(hypot(alpha, sqrt(ss)), alpha);
@@ -334,8 +358,9 @@ __device__ __forceinline__ double tl_reduce8(const double (&x)[8])
 	return d;
 }
 
+// (at most 128 registers: a SIMD holds four waves, 512 threads' or less workgroups a sample each)
 template <int BT, int RPT, int NB>
-__global__ __launch_bounds__(BT) void tl_tridiag_panel_kernel(double *__restrict__ Aall, unsigned n, double *__restrict__ dall,
+__global__ __launch_bounds__(BT) __attribute__((amdgpu_waves_per_eu(4))) void tl_tridiag_panel_kernel(double *__restrict__ Aall, unsigned n, double *__restrict__ dall,
 		double *__restrict__ eall, double *__restrict__ tall)
 {
 	extern __shared__ double sh[];
@@ -1083,7 +1108,7 @@ __global__ __launch_bounds__(256) void tl_back_kernel(const double *__restrict__
 constexpr int TL_WB = 32;        // reflectors per block
 constexpr int TL_WC = 16;        // columns of Z per workgroup
 constexpr int TL_WW = 8;         // waves per workgroup
-constexpr int TL_WRB = 8;        // 16-row blocks per wave (8 waves: N <= 1024)
+constexpr int TL_WRB = 8;        // most 16-row blocks per wave (8 waves: N <= 1024)
 
 // Yb[b][r][k] = v_{32 b + k}[r]: the reflectors of each block as a row-major panel of n16 =
 // 16 ceil(N / 16) rows x 32 (zero outside their support and in the padding rows), so that a row's
@@ -1160,16 +1185,17 @@ __global__ __launch_bounds__(256) void tl_wy_t_kernel(const double *__restrict__
 	for(unsigned e = tid; e < TL_WB * TL_WB; e += 256) To[e] = T[e / TL_WB][e % TL_WB];
 }
 
-// Z <- Q Z for 16 columns per workgroup (grid (N / 16, samples)), N <= 1024.  Wave w of the 8 holds
-// rows 128 w .. 128 w + 127 of its columns in the matrix-core accumulator layout (16 x 16 blocks: lane
+// Z <- Q Z for 16 columns per workgroup (tl_item), N <= 128 RB.  Wave w of the 8 holds
+// the 16 RB rows from 16 RB w of its columns in the matrix-core accumulator layout (16 x 16 blocks: lane
 // l, element e = row 4 e + l / 16, column l % 16) for the whole sweep over the blocks, so Z is read
 // and written once.  Per block: W^T = Z^T Y (each wave over its rows; the accumulator elements
 // serve directly as the A operand, rows 16 q + 4 e + l / 16 of step (q, e)), the eight waves'
 // parts summed in LDS, W2^T = W^T T^T, then Z -= Y W2 (v_mfma_f64_16x16x4 both ways).  Z comes as [row][column]
 // with 1 / |column| in rn from the twisted factorisations, or by columns from the QL iteration (ql[s]);
 // V is written by columns.
+template <int RB>
 __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *__restrict__ Yball, const double *__restrict__ Tall,
-		unsigned n, unsigned nblk, const double *__restrict__ Zall, const double *__restrict__ rnall, const int *__restrict__ ql,
+		unsigned n, unsigned ns, unsigned nblk, const double *__restrict__ Zall, const double *__restrict__ rnall, const int *__restrict__ ql,
 		double *__restrict__ Vall)
 {
 	typedef double v4d __attribute__((ext_vector_type(4)));
@@ -1177,18 +1203,20 @@ __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *_
 	__shared__ double wpart[TL_WW][2][64][4];
 	__shared__ double Wt[TL_WC][TL_WB + 1];
 	__shared__ double W2t[TL_WC][TL_WB + 1];
-	const unsigned s = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-	const unsigned g = lane >> 4, m = lane & 15, c0 = blockIdx.x * TL_WC, n16 = (n + 15) & ~15u;
+	unsigned s, item;
+	tl_item(blockIdx.x, (n + TL_WC - 1) / TL_WC, ns, s, item);
+	const unsigned tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+	const unsigned g = lane >> 4, m = lane & 15, c0 = item * TL_WC, n16 = (n + 15) & ~15u;
 	const double *Tb = Tall + (size_t)s * nblk * TL_WB * TL_WB;
 	const double *Z = Zall + (size_t)s * n * n;
 	double *V = Vall + (size_t)s * n * n;
-	const unsigned rw0 = wave * 16 * TL_WRB;                      // first row of this wave
+	const unsigned rw0 = wave * 16 * RB;                      // first row of this wave
 	const unsigned col = c0 + m;
 	const bool by_col = ql[s] != 0;
 	const double rn = by_col || col >= n ? 1.0 : rnall[(size_t)s * n + col];
-	v4d acc[TL_WRB];
+	v4d acc[RB];
 #pragma unroll
-	for(int q = 0; q < TL_WRB; q++)
+	for(int q = 0; q < RB; q++)
 #pragma unroll
 		for(int e = 0; e < 4; e++){
 			const unsigned r = rw0 + 16 * q + 4 * e + g;
@@ -1204,7 +1232,7 @@ __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *_
 		// W^T partial over this wave's rows r >= jb + 1 (Y is zero above)
 		v4d wt[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
-		for(int q = 0; q < TL_WRB; q++){
+		for(int q = 0; q < RB; q++){
 			const unsigned rb = rw0 + 16 * q;
 			if(rb + 16 <= jb + 1 || rb >= n) continue;           // uniform per wave
 #pragma unroll
@@ -1243,7 +1271,7 @@ __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *_
 		// Z[rows][cols] -= Y[rows][k] W2[k][cols]: A = Y (row 16 q + l % 16, k 4 t + l / 16), B = -W2
 		// (k 4 t + l / 16, column l % 16)
 #pragma unroll
-		for(int q = 0; q < TL_WRB; q++){
+		for(int q = 0; q < RB; q++){
 			const unsigned rb = rw0 + 16 * q;
 			if(rb + 16 <= jb + 1 || rb >= n) continue;
 #pragma unroll
@@ -1254,7 +1282,7 @@ __global__ __launch_bounds__(64 * TL_WW) void tl_wy_apply_kernel(const double *_
 		}
 	}
 #pragma unroll
-	for(int q = 0; q < TL_WRB; q++)
+	for(int q = 0; q < RB; q++)
 #pragma unroll
 		for(int e = 0; e < 4; e++){
 			const unsigned r = rw0 + 16 * q + 4 * e + g;
@@ -1325,7 +1353,7 @@ __global__ __launch_bounds__(256) void tl_current_kernel(const double *__restric
 }
 
 // ---- pair tiles: J_c(j, i) = v_j . W_c[:, i], binned --------------------------------------
-// grid (i-block, j-block, sample), 64 x 64 tiles, 4 waves.  The tile is a GEMM over the N rows:
+// (i-block, j-block, sample) by tl_item, 64 x 64 tiles, 4 waves.  The tile is a GEMM over the N rows:
 // wave w computes the 32 x 32 quarter (j: 32 (w / 2), i: 32 (w % 2)) of J_0 and J_1 with
 // v_mfma_f64_16x16x4_f64, 2 x 2 blocks of 16 x 16, from 16-row panels of V, W_0, W_1 staged in
 // LDS.  Operand layout of the instruction: A[m][k] in lane m + 16 k, B[k][n] in lane n + 16 k,
@@ -1334,15 +1362,21 @@ typedef double tl_v4d __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256) void tl_pairs_kernel(const double *__restrict__ Vall, const double *__restrict__ W0all,
 		const double *__restrict__ W1all, const double *__restrict__ evs_all, const double *__restrict__ ems_all,
-		unsigned n, double width, unsigned nbins, double *__restrict__ part)
+		unsigned n, unsigned ns, double width, unsigned nbins, double *__restrict__ part)
 {
-	__shared__ double Vs[TL_KC][TL_TILE + 1], W0s[TL_KC][TL_TILE + 1], W1s[TL_KC][TL_TILE + 1];
-	__shared__ unsigned ebin[TL_TILE * TL_TILE];
-	__shared__ double eval[TL_TILE * TL_TILE];
+	// rows of bins one place apart in the banks; the stages of V, W_0, W_1 reuse the bins' and values' space
+	constexpr unsigned LD = TL_TILE + 1;
+	__shared__ double eval[TL_TILE * LD];
+	__shared__ unsigned ebin[TL_TILE * LD];
 	__shared__ unsigned brange[2];
 	__shared__ uint2 rrange[TL_TILE];
-	__shared__ double hacc[TL_HB];
-	const unsigned ib = blockIdx.x, jb = blockIdx.y, s = blockIdx.z, nblk = gridDim.x;
+	__shared__ double hacc[4][TL_HB];
+	static_assert(3 * TL_KC * LD <= TL_TILE * LD, "stages fit the values");
+	double (*Vs)[LD] = reinterpret_cast<double (*)[LD]>(eval), (*W0s)[LD] = Vs + TL_KC, (*W1s)[LD] = W0s + TL_KC;
+	const unsigned nblk = (n + TL_TILE - 1) / TL_TILE;
+	unsigned s, item;
+	tl_item(blockIdx.x, nblk * nblk, ns, s, item);
+	const unsigned ib = item % nblk, jb = item / nblk;
 	const unsigned tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 	const unsigned i0 = ib * TL_TILE, j0 = jb * TL_TILE;
 	const double *evs = evs_all + (size_t)s * n, *ems = ems_all + (size_t)s * n;
@@ -1435,8 +1469,8 @@ __global__ __launch_bounds__(256) void tl_pairs_kernel(const double *__restrict_
 						bmax = max(bmax, bin);
 					}
 				}
-				ebin[jl * TL_TILE + il] = bin;
-				eval[jl * TL_TILE + il] = val;
+				ebin[jl * LD + il] = bin;
+				eval[jl * LD + il] = val;
 			}
 	if(bmin != TL_NONE){
 		atomicMin(&brange[0], bmin);
@@ -1447,7 +1481,7 @@ __global__ __launch_bounds__(256) void tl_pairs_kernel(const double *__restrict_
 	// the last bin), then non-increasing, then TL_NONE (E_i > E_j or i >= n): each bin is one run
 	// per row.  Row ranges first, then the runs are added to their bins row by row.
 	if(tid < TL_TILE){
-		const unsigned *rb = ebin + tid * TL_TILE;
+		const unsigned *rb = ebin + tid * LD;
 		unsigned lo = TL_TILE, hi = 0;
 		for(unsigned il = 0; il < TL_TILE; il++)
 			if(rb[il] != TL_NONE){
@@ -1460,26 +1494,31 @@ __global__ __launch_bounds__(256) void tl_pairs_kernel(const double *__restrict_
 	const unsigned blo = brange[0], bhi = brange[1];
 	if(blo != TL_NONE && bhi - blo < TL_HB){
 		// A row's runs fall in distinct bins, so one wave adds the runs of row after row (the LDS
-		// operations of a wave complete in order): every bin adds its rows' run sums in row order,
-		// each run summed with i ascending.
-		for(unsigned b = tid; b < TL_HB; b += 256) hacc[b] = 0;
+		// operations of a wave complete in order).  Wave w takes the tile's rows 16 w .. 16 w + 15 into
+		// a histogram of its own: every bin adds its rows' run sums in row order, each run summed with
+		// i ascending, then the four waves' sums in order.  (One wave for all 64 rows kept the other
+		// three waiting: 28.5 against 23.9 ms for 256 samples at N = 1024.)
+		for(unsigned b = tid; b < 4 * TL_HB; b += 256) hacc[0][b] = 0;
 		__syncthreads();
-		if(wave == 0)
-			for(unsigned jl = 0; jl < TL_TILE; jl++){
-				const uint2 rr = rrange[jl];
-				const unsigned *rb = ebin + jl * TL_TILE;
-				const unsigned il = lane;
-				if(il >= rr.x && il < rr.y){
-					const unsigned bin = rb[il];
-					if(bin != TL_NONE && (il == rr.x || rb[il - 1] != bin)){
-						double sum = 0;
-						for(unsigned q = il; q < rr.y && rb[q] == bin; q++) sum += eval[jl * TL_TILE + q];
-						hacc[bin - blo] += sum;
-					}
+		for(unsigned jl = 16 * wave; jl < 16 * wave + 16; jl++){
+			const uint2 rr = rrange[jl];
+			const unsigned *rb = ebin + jl * LD;
+			const unsigned il = lane;
+			if(il >= rr.x && il < rr.y){
+				const unsigned bin = rb[il];
+				if(bin != TL_NONE && (il == rr.x || rb[il - 1] != bin)){
+					double sum = 0;
+					for(unsigned q = il; q < rr.y && rb[q] == bin; q++) sum += eval[jl * LD + q];
+					hacc[wave][bin - blo] += sum;
 				}
 			}
+		}
 		__syncthreads();
-		for(unsigned b = tid; b < nbins; b += 256) out[b] = (b >= blo && b <= bhi) ? hacc[b - blo] : 0.0;
+		for(unsigned b = tid; b < nbins; b += 256){
+			double t = 0;
+			if(b >= blo && b <= bhi) t = ((hacc[0][b - blo] + hacc[1][b - blo]) + hacc[2][b - blo]) + hacc[3][b - blo];
+			out[b] = t;
+		}
 		return;
 	}
 	// wide tiles: every bin finds its run in each row by binary search and adds it row by row
@@ -1489,7 +1528,7 @@ __global__ __launch_bounds__(256) void tl_pairs_kernel(const double *__restrict_
 			for(unsigned jl = 0; jl < TL_TILE; jl++){
 				const uint2 rr = rrange[jl];
 				if(rr.x >= rr.y) continue;
-				const unsigned *rb = ebin + jl * TL_TILE;
+				const unsigned *rb = ebin + jl * LD;
 				if(b > rb[rr.x] || b < rb[rr.y - 1]) continue;
 				// first il with bin <= b, then first il with bin < b
 				unsigned p = rr.x, q = rr.y;
@@ -1504,7 +1543,7 @@ __global__ __launch_bounds__(256) void tl_pairs_kernel(const double *__restrict_
 					if(rb[mid] < b) u = mid;
 					else t = mid + 1;
 				}
-				for(unsigned il = p; il < t; il++) sum += eval[jl * TL_TILE + il];
+				for(unsigned il = p; il < t; il++) sum += eval[jl * LD + il];
 			}
 		out[b] = sum;
 	}
@@ -1612,8 +1651,7 @@ extern "C" int ephmc_tl_hist(ephmc_ctx *c, const double *normals, unsigned nsamp
 	const size_t mat = (size_t)n * n;
 	const unsigned nblk = (n + TL_TILE - 1) / TL_TILE;
 	// samples per batch: about 100 GB of workspace (5.5 N^2 doubles per sample; EPHMC_TL_BATCH_MB
-	// sets another budget in MiB), at most 2048, so that the one-wave-per-sample QL recurrence has
-	// two waves on every SIMD
+	// sets another budget in MiB), at most 2048, which fill every kernel's grid several times over
 	size_t mb = (size_t)100 << 10;
 	if(const char *v = getenv("EPHMC_TL_BATCH_MB")) mb = std::max<size_t>(1, strtoull(v, nullptr, 10));
 	const size_t per = (size_t)(5.5 * mat * 8) + (size_t)nblk * nblk * nbins * 8;
@@ -1638,10 +1676,19 @@ extern "C" int ephmc_tl_hist(ephmc_ctx *c, const double *normals, unsigned nsamp
 		EPHMC_TRY(timer_begin(c, "tl_tridiag"));
 		{
 			if(n <= TL_BT){
-				const size_t lds = tl_panel_lds_doubles<TL_BT, TL_PNB>(n) * 8;
-				(void)hipFuncSetAttribute((const void *)tl_tridiag_panel_kernel<TL_BT, 1, TL_PNB>,
-					hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-				tl_tridiag_panel_kernel<TL_BT, 1, TL_PNB><<<nb_, TL_BT, lds, c->stream>>>(w.A, n, w.d, w.e, w.tau);
+				// a thread per row: the smallest workgroup that has them, so that a CU holds several samples
+#define EPHMC_TRIDIAG(BT)                                                                              \
+				do {                                                                                    \
+					const size_t lds = tl_panel_lds_doubles<BT, TL_PNB>(n) * 8;                          \
+					(void)hipFuncSetAttribute((const void *)tl_tridiag_panel_kernel<BT, 1, TL_PNB>,      \
+						hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                           \
+					tl_tridiag_panel_kernel<BT, 1, TL_PNB><<<nb_, BT, lds, c->stream>>>(w.A, n, w.d, w.e, w.tau); \
+				} while(0)
+				if(n <= 128) EPHMC_TRIDIAG(128);
+				else if(n <= 256) EPHMC_TRIDIAG(256);
+				else if(n <= 512) EPHMC_TRIDIAG(512);
+				else EPHMC_TRIDIAG(TL_BT);
+#undef EPHMC_TRIDIAG
 			}else{
 				const size_t lds = (3 * (size_t)n + TL_BT / 64) * 8;
 				if(n <= TL_BT) tl_tridiag_kernel<TL_BT, 1><<<nb_, TL_BT, lds, c->stream>>>(w.A, n, w.d, w.e, w.tau);
@@ -1685,7 +1732,10 @@ extern "C" int ephmc_tl_hist(ephmc_ctx *c, const double *normals, unsigned nsamp
 			tl_wy_t_kernel<<<dim3(nblkw, nb_), 256, 0, c->stream>>>(w.A, w.tau, n, tall);
 			EPHMC_LAUNCHED();
 			// (the reflectors' copy is made: A takes the vectors)
-			tl_wy_apply_kernel<<<dim3((n + TL_WC - 1) / TL_WC, nb_), 64 * TL_WW, 0, c->stream>>>(yball, tall, n, nblkw, w.Z, w.rn, w.ql, w.A);
+			const unsigned wg = (n + TL_WC - 1) / TL_WC * nb_;
+			if(n <= 256) tl_wy_apply_kernel<2><<<wg, 64 * TL_WW, 0, c->stream>>>(yball, tall, n, nb_, nblkw, w.Z, w.rn, w.ql, w.A);
+			else if(n <= 512) tl_wy_apply_kernel<4><<<wg, 64 * TL_WW, 0, c->stream>>>(yball, tall, n, nb_, nblkw, w.Z, w.rn, w.ql, w.A);
+			else tl_wy_apply_kernel<TL_WRB><<<wg, 64 * TL_WW, 0, c->stream>>>(yball, tall, n, nb_, nblkw, w.Z, w.rn, w.ql, w.A);
 			vec = w.A;
 		}else if(n <= 1024) tl_back_kernel<16, 4><<<dim3((n + 15) / 16, nb_), 256, 0, c->stream>>>(w.A, w.tau, w.Z, n);
 		else tl_back_kernel<32, 2><<<dim3((n + 7) / 8, nb_), 256, 0, c->stream>>>(w.A, w.tau, w.Z, n);
@@ -1699,7 +1749,7 @@ extern "C" int ephmc_tl_hist(ephmc_ctx *c, const double *normals, unsigned nsamp
 			contr_mat[3], contr_mat[4], contr_mat[5], sorted, w.W0, w.W1);
 		EPHMC_LAUNCHED();
 		EPHMC_TRY(timer_begin(c, "tl_pairs"));
-		tl_pairs_kernel<<<dim3(nblk, nblk, nb_), 256, 0, c->stream>>>(sorted, w.W0, w.W1, w.evs, w.ems, n, width, nbins, w.part);
+		tl_pairs_kernel<<<nblk * nblk * nb_, 256, 0, c->stream>>>(sorted, w.W0, w.W1, w.evs, w.ems, n, nb_, width, nbins, w.part);
 		EPHMC_LAUNCHED();
 		{
 			const unsigned nparts = nb_ * nblk * nblk, nch = (nparts + TL_RC - 1) / TL_RC;

@@ -161,3 +161,21 @@ def test_tl_degenerate_pairs(l1, l2, scale):
     gr, zr = sum(r[0] for r in ref), np.array([r[1] for r in ref])
     assert np.abs(z / zr - 1).max() < 1e-12
     assert rel(g[1:], gr[1:]) < 1e-9
+
+
+@pytest.mark.parametrize("l1,l2", [(8, 16), (16, 16), (20, 25)])
+def test_tl_many_samples_repeatable(l1, l2):
+    """Several samples' workgroups on a CU at once (128, 256 and 512 threads each): the same bits in every
+    run, and the partition sums of the last samples against LAPACK."""
+    nbins, ns = 64, 1024
+    om, width = tl_model(l1, l2, nbins)
+    xs = draws(om, ns, 77)
+    say("tl repeatable", l1, l2)
+    ctx = gpu_context(om)
+    runs = [ctx.tl_hist(xs, CM, width, nbins) for _ in range(3)]
+    for g, z in runs[1:]:
+        np.testing.assert_array_equal(z, runs[0][1])
+        np.testing.assert_array_equal(g, runs[0][0])
+    for q in range(ns - 8, ns):
+        E = np.linalg.eigvalsh(D.hopping_matrix(om.nnt, om.ns, xs[q], om.t, om.kappa, -om.mu))
+        assert abs(runs[0][1][q] / (np.exp(-E).sum() / om.ns) - 1) < 1e-12
