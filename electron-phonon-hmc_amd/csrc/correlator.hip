@@ -9,22 +9,42 @@
 //   g_ab(tau) = 1/N sum_{i,j} chi_ia chi_jb [R_t0[j*N+i] R_0t[jb*N+ia] + R_t0[jb*N+ia] R_0t[j*N+i]
 //                                        - R_t0[jb*N+i] R_0t[j*N+ia] - R_t0[j*N+ia] R_0t[jb*N+i]]
 // with ia = nb(i, 2a), jb = nb(j, 2b), chi_ia = t_a - kappa_a x[0][i][a], chi_jb from slice tau.
-// One launch covers every tau: a workgroup takes a chunk of j for one tau and, for each j, stages
-// the rows j and jb (b = 0..2) of both propagators in LDS, from where its threads gather the
-// entries at i and ia; block sums per (tau, j-chunk), then a fixed-order pass per tau.
+// With the antisymmetric current matrices J_a = sum_i chi_ia (|i><ia| - |ia><i|) of slice 0 and J'_b of
+// slice tau, and R_0t as the row-indexed Q[j][i] = R_0t[j*N+i], that sum is
+//   g_ab(tau) = -1/N sum_{i,j} (J_a R_t0)[i][j] (J'_b Q)[j][i]:
+// two neighbours of i in R_t0's column j per a, two neighbours of j in Q's rows per b, then nine
+// products, in place of four products of gathered entries for each of the nine (a, b).
+// One launch covers every tau.  A workgroup takes up to CC_L sites j of a lattice row (of CC_R rows
+// where rows are short) and walks them in order: R_t0's column goes through LDS for the neighbours in
+// i, the rows of Q slide along in registers (three new ones per j), all loaded one j ahead.  Block
+// sums per (tau, workgroup), then a fixed-order pass per tau.
 #include "internal.h"
 #include "alloc_group.h"
 #include <mutex>
 
 namespace ephmc {
 
-constexpr int CC_BT = 1024;
-constexpr unsigned CC_J = 8;   // values of j per workgroup
+constexpr unsigned CC_L = 32;  // sites j of one lattice row per workgroup
+constexpr unsigned CC_J = 8;   // (sizes the block sums: at least this many sites j per workgroup)
 
-// block sums of one correlator call: [nt][ceil(N/CC_J)][9]
+// block sums of one correlator call: at most [nt][ceil(N/CC_J)][9]
 static size_t cc_partials(unsigned ns, unsigned nt)
 {
 	return (size_t)nt * ((ns + CC_J - 1) / CC_J) * 9;
+}
+
+// workgroups per slice: pieces of a lattice row times row groups, with at least CC_J sites j each
+// (but for the last), so no more than ceil(N / CC_J)
+struct CcShape { unsigned pieces, len, rows, groups; };
+
+static CcShape cc_shape(const ephmc_ctx *c)
+{
+	CcShape s;
+	s.pieces = (c->l1 + CC_L - 1) / CC_L;
+	s.len = (c->l1 + s.pieces - 1) / s.pieces;
+	s.rows = c->l1 < CC_J ? (CC_J + c->l1 - 1) / c->l1 : 1;
+	s.groups = (c->l2 + s.rows - 1) / s.rows;
+	return s;
 }
 
 // R_t0 and R_0t (store values each) and the result block (res values), all or none
@@ -46,65 +66,107 @@ static int cc_alloc(ephmc_ctx *c, size_t store, size_t res)
 	return EPHMC_OK;
 }
 
-// grid (j-chunks of CC_J, tau).  rows (dynamic LDS, 8 N doubles): R_t0[j], R_0t[j], R_t0[jb]
-// (b = 0..2), R_0t[jb] (b = 0..2); thread t takes the sites i = t, t + CC_BT, ...
-__global__ __launch_bounds__(CC_BT) void cc_contract_kernel(const double *__restrict__ Tfin, const double *__restrict__ Rt0,
-		const double *__restrict__ R0t, const double *__restrict__ x, const int *__restrict__ nb, double t0, double t1, double t2,
-		double k0, double k1, double k2, unsigned ns, unsigned nt, double *__restrict__ partial)
+// a b - c d with both products rounded: exactly zero where they are equal (lattices of extent 1)
+__device__ __forceinline__ double cc_diff(double a, double b, double c, double d)
 {
-	extern __shared__ double rows[];
-	__shared__ double red[9][CC_BT / 64];
-	const double tk[3] = {t0, t1, t2}, kk[3] = {k0, k1, k2};
-	const unsigned tau = blockIdx.y;
+#pragma clang fp contract(off)
+	return a * b - c * d;
+}
+
+// Thread t takes the sites i = t + BT q, q < S (BT S >= N).  Workgroup b: slice and item by cc_item.
+// What bounds it: the 2 nt N^2 values read from memory once (2 GB at 32x32, nt 128); each piece's first and
+// last columns and the rows above and below it come a second and third time, from the XCD's L2, to
+// which all workgroups of a slice go.  585 us there, 3.6 TB/s; with the gathered entries of all nine
+// (a, b) from eight rows in LDS 1975 us.
+template <int BT, int S>
+__global__ __launch_bounds__(BT) void cc_contract_kernel(const double *__restrict__ Tfin, const double *__restrict__ Rt0,
+		const double *__restrict__ R0t, const double *__restrict__ coef, const int *__restrict__ nb, unsigned ns, unsigned nt,
+		unsigned l1, unsigned l2, CcShape sh, double *__restrict__ partial)
+{
+	extern __shared__ double rows[];                 // 2 ns: column j of R_t0, by parity of the step
+	__shared__ double red[9][BT / 64];
+	// eight slices at a time, one to an XCD (workgroups go to the XCDs in turn)
+	const unsigned per = sh.pieces * sh.groups, full = nt / 8 * 8, b = blockIdx.x;
+	const unsigned tau = b < full * per ? b / (8 * per) * 8 + b % 8 : full + (b - full * per) / per;
+	const unsigned item = b < full * per ? b / 8 % per : (b - full * per) % per;
 	const size_t mat = (size_t)ns * ns;
 	const double *rt = tau == 0 ? Tfin : Rt0 + (size_t)(nt - tau) * mat;
 	const double *r0 = R0t + (size_t)tau * mat;
-	const double *xt = x + (size_t)tau * 3 * ns;
+	const double *ct = coef + (size_t)tau * 6 * ns;
+	unsigned site[S];
+	int in[S][6];
+	double cf[S][6];
+#pragma unroll
+	for(int q = 0; q < S; q++){
+		// a thread past the last site works on it with zero coefficients
+		const unsigned i = threadIdx.x + BT * q;
+		site[q] = min(i, ns - 1);
+#pragma unroll
+		for(int d = 0; d < 6; d++){
+			in[q][d] = nb[d * ns + site[q]];
+			cf[q][d] = i < ns ? coef[d * ns + site[q]] : 0.0;
+		}
+	}
 	double g[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-	const unsigned j0 = blockIdx.x * CC_J, j1 = min(j0 + CC_J, ns);
-	for(unsigned j = j0; j < j1; j++){
-		unsigned jb[3];
-		double chijb[3];
+	const unsigned xa = item % sh.pieces * sh.len, xe = min(xa + sh.len, l1);
+	unsigned step = 0;
+	for(unsigned y = item / sh.pieces * sh.rows; y < min(item / sh.pieces * sh.rows + sh.rows, l2); y++){
+		const double *qc = r0 + (size_t)y * l1 * ns, *qu = r0 + (size_t)((y + 1) % l2) * l1 * ns,
+			*qd = r0 + (size_t)((y + l2 - 1) % l2) * l1 * ns, *pc = rt + (size_t)y * l1 * ns;
+		auto col = [&](const double *m, unsigned x, int q){ return m[(size_t)x * ns + site[q]]; };
+		// Q's rows around j = (x, y): c0, c1 = x - 1, x; c2 = x + 1 (the row above: u0, u1 = x - 1, x; below:
+		// d1, d2 = x, x + 1)
+		double c0[S], c1[S], c2[S], u0[S], u1[S], d1[S], d2[S], p[S];
 #pragma unroll
-		for(int b = 0; b < 3; b++){
-			jb[b] = (unsigned)nb[(2 * b) * ns + j];
-			chijb[b] = tk[b] - kk[b] * xt[(size_t)j * 3 + b];
+		for(int q = 0; q < S; q++){
+			c0[q] = col(qc, (xa + l1 - 1) % l1, q);
+			c1[q] = col(qc, xa, q);
+			c2[q] = col(qc, (xa + 1) % l1, q);
+			u0[q] = col(qu, (xa + l1 - 1) % l1, q);
+			u1[q] = col(qu, xa, q);
+			d1[q] = col(qd, xa, q);
+			d2[q] = col(qd, (xa + 1) % l1, q);
+			p[q] = col(pc, xa, q);
 		}
-		__syncthreads();                 // the previous j's rows are no longer read
-		for(unsigned i = threadIdx.x; i < ns; i += CC_BT){
-			rows[i] = rt[(size_t)j * ns + i];
-			rows[ns + i] = r0[(size_t)j * ns + i];
+		for(unsigned x = xa; x < xe; x++, step++){
+			double *row = rows + (step & 1) * ns;
 #pragma unroll
-			for(int b = 0; b < 3; b++){
-				rows[(2 + b) * ns + i] = rt[(size_t)jb[b] * ns + i];
-				rows[(5 + b) * ns + i] = r0[(size_t)jb[b] * ns + i];
-			}
-		}
-		__syncthreads();
-		for(unsigned i = threadIdx.x; i < ns; i += CC_BT){
-			const double rt_ji = rows[i], r0_ji = rows[ns + i];
-			unsigned ia[3];
-			double chia[3], rt_jia[3], r0_jia[3];
+			for(int q = 0; q < S; q++) row[site[q]] = p[q];
+			const unsigned j = y * l1 + x, x1 = (x + 1) % l1, x2 = (x + 2) % l1;
+			double cj[6];
 #pragma unroll
-			for(int a = 0; a < 3; a++){
-				ia[a] = (unsigned)nb[(2 * a) * ns + i];
-				chia[a] = tk[a] - kk[a] * x[(size_t)i * 3 + a];
-				rt_jia[a] = rows[ia[a]];
-				r0_jia[a] = rows[ns + ia[a]];
+			for(int d = 0; d < 6; d++) cj[d] = ct[d * ns + j];
+			__syncthreads();
+			// the next j's new values (its row of the other parity was last read before this barrier)
+			double nc[S], nu[S], nd[S], np[S];
+#pragma unroll
+			for(int q = 0; q < S; q++){
+				nc[q] = col(qc, x2, q);
+				nu[q] = col(qu, x1, q);
+				nd[q] = col(qd, x2, q);
+				np[q] = col(pc, x1, q);
 			}
 #pragma unroll
-			for(int b = 0; b < 3; b++){
-				const double *rtb = rows + (2 + b) * ns, *r0b = rows + (5 + b) * ns;
-				const double rt_jbi = rtb[i], r0_jbi = r0b[i];
+			for(int q = 0; q < S; q++){
+				double f[3], h[3];
 #pragma unroll
-				for(int a = 0; a < 3; a++){
-					const double rt_jbia = rtb[ia[a]], r0_jbia = r0b[ia[a]];
-					double corr = rt_ji * r0_jbia;
-					corr += rt_jbia * r0_ji;
-					corr -= rt_jbi * r0_jia[a];
-					corr -= rt_jia[a] * r0_jbi;
-					g[a * 3 + b] += chia[a] * chijb[b] * corr;
-				}
+				for(int a = 0; a < 3; a++) f[a] = cc_diff(cf[q][2 * a], row[in[q][2 * a]], cf[q][2 * a + 1], row[in[q][2 * a + 1]]);
+				// neighbours of j: right / left, up / down, up-left / down-right
+				h[0] = cc_diff(cj[0], c2[q], cj[1], c0[q]);
+				h[1] = cc_diff(cj[2], u1[q], cj[3], d1[q]);
+				h[2] = cc_diff(cj[4], u0[q], cj[5], d2[q]);
+#pragma unroll
+				for(int a = 0; a < 3; a++)
+#pragma unroll
+					for(int bb = 0; bb < 3; bb++) g[a * 3 + bb] = fmac(f[a], h[bb], g[a * 3 + bb]);
+				c0[q] = c1[q];
+				c1[q] = c2[q];
+				c2[q] = nc[q];
+				u0[q] = u1[q];
+				u1[q] = nu[q];
+				d1[q] = d2[q];
+				d2[q] = nd[q];
+				p[q] = np[q];
 			}
 		}
 	}
@@ -120,8 +182,8 @@ __global__ __launch_bounds__(CC_BT) void cc_contract_kernel(const double *__rest
 	__syncthreads();
 	if(threadIdx.x < 9){
 		double t = 0;
-		for(int w = 0; w < CC_BT / 64; w++) t += red[threadIdx.x][w];
-		partial[((size_t)tau * gridDim.x + blockIdx.x) * 9 + threadIdx.x] = t;
+		for(int w = 0; w < BT / 64; w++) t += red[threadIdx.x][w];
+		partial[((size_t)tau * per + item) * 9 + threadIdx.x] = -t;
 	}
 }
 
@@ -155,12 +217,22 @@ static int correlate(ephmc_ctx *c, const double *x, const double *minv, double l
 	// R_0t: transposed inverse, then slices 0 .. nt-1 ascending; stored entry tau = state at tau
 	if(!ident) EPHMC_TRY(transpose_plus_identity(c, EPHMC_FP64, minv, c->d_gj[0], 0));
 	EPHMC_TRY(chain_forward(c, EPHMC_FP64, c->d_gj[0], c->d_gj[1], R0t, 1, 0, ident));
-	const unsigned by = (ns + CC_J - 1) / CC_J;
-	const size_t lds = 8 * (size_t)ns * sizeof(double);
-	if(lds + 9 * (CC_BT / 64) * sizeof(double) > 160 * 1024){ set_error("correlator: %u sites exceed the LDS", ns); return EPHMC_ERR_UNSUPPORTED; }
-	(void)hipFuncSetAttribute((const void *)cc_contract_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-	cc_contract_kernel<<<dim3(by, nt), CC_BT, lds, c->stream>>>(c->d_Tfin, Rt0, R0t, x, c->d_nb,
-		c->cfg.t[0], c->cfg.t[1], c->cfg.t[2], c->cfg.kappa[0], c->cfg.kappa[1], c->cfg.kappa[2], ns, nt, partial);
+	const CcShape sh = cc_shape(c);
+	const unsigned by = sh.pieces * sh.groups;
+	const size_t lds = 2 * (size_t)ns * sizeof(double);
+#define EPHMC_CC(BT, S)                                                                                    \
+	cc_contract_kernel<BT, S><<<by * nt, BT, lds, c->stream>>>(c->d_Tfin, Rt0, R0t, c->d_coef64, c->d_nb, ns, nt, c->l1, \
+		c->l2, sh, partial)
+	// two sites i per thread, so that a CU holds workgroups enough to cover each other's barriers
+	// (32x32: 585 us against 830 with one site on 1024 threads)
+	if(ns <= 64) EPHMC_CC(64, 1);
+	else if(ns <= 128) EPHMC_CC(64, 2);
+	else if(ns <= 256) EPHMC_CC(128, 2);
+	else if(ns <= 512) EPHMC_CC(256, 2);
+	else if(ns <= 1024) EPHMC_CC(512, 2);
+	else if(ns <= 2048) EPHMC_CC(512, 4);
+	else { set_error("correlator: %u sites exceed 2048", ns); return EPHMC_ERR_UNSUPPORTED; }
+#undef EPHMC_CC
 	EPHMC_LAUNCHED();
 	cc_sum_kernel<<<nt, 576, 0, c->stream>>>(partial, by, c->cfg.single_particle ? exp(-logdet) : 1.0 / ns,
 		out);

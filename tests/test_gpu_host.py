@@ -32,6 +32,24 @@ def oracle_greens(om, x, Minv, ld):
     return g.reshape(nt, 3, 3)
 
 
+# lattices of one row or column and of short rows (several rows per workgroup), rows of more than one
+# piece (33, 40), slice counts around a multiple of eight, every workgroup shape up to N = 1056
+@pytest.mark.parametrize("l1,l2,nt", [(1, 1, 3), (1, 9, 2), (9, 1, 8), (2, 2, 9), (3, 7, 5), (5, 25, 4), (33, 3, 9), (40, 2, 3), (16, 16, 8),
+                                      (17, 30, 2), (23, 31, 3), (33, 32, 2)])
+def test_cc_correlator_shapes(l1, l2, nt):
+    say("cc_correlator", l1, l2, nt)
+    om = OracleModel(l1, l2, nt, beta=nt * 40 / 32)
+    ctx = gpu_context(om)
+    n = om.ns
+    x = np.random.default_rng(l1 + l2).standard_normal(om.dim) * 0.5
+    ld, _, Minv = om.logdet_inv(om.M_hat(x))
+    go = np.zeros(nt * 9)
+    oracle().orc_cc_correlator(om.ref, ptr(x), ptr(Minv), ptr(np.zeros(nt * n * n)), ptr(np.zeros(n * n)), ptr(np.zeros(2 * n * n)),
+                               ptr(go), ld)
+    g = ctx.cc_correlator(x, Minv, ld)
+    assert np.abs(g.ravel() - go).max() <= 1e-10 * max(np.abs(go).max(), 1e-30)
+
+
 @pytest.mark.parametrize("l1,l2,nt", [(1, 4, 4), (2, 3, 8), (4, 4, 8), (6, 6, 16), (5, 7, 12)])
 def test_cc_correlator(l1, l2, nt):
     say("cc_correlator", l1, l2, nt)
