@@ -5,7 +5,10 @@
 // workgroup loads LW complex series into LDS (z[t][l], links contiguous, coalesced rows),
 // transforms them (radix-2 decimation in frequency: natural order in, bit-reversed modes out),
 // applies the per-mode operation, and transforms back (decimation in time: bit-reversed in,
-// natural out), so no permutation pass is needed.  Non-power-of-two nt uses direct sums.
+// natural out), so no permutation pass is needed.  Two radix-2 stages run in one pass over LDS.
+// Non-power-of-two nt uses direct sums.  Bound by LDS latency and barriers (8 passes at nt = 128) and the
+// launch: momentum refresh and drift at 32x32, nt 128 19.5 us together (stage by stage 27.1, with a runtime
+// division per butterfly); nt 95 27 us (63 with a 64-bit remainder per term).
 // Two real series share one complex transform:
 //   evolve:  z = x + i p of one link; with X_n = (Z_n + conj Z_-n)/2, P_n = (Z_n - conj Z_-n)/2i
 //            the exact flow X' = cos h X + sin h P/f_n, P' = cos h P - sin h f_n X per mode
@@ -41,7 +44,13 @@ struct FftArgs {
 	int mode;
 };
 
-__device__ __forceinline__ double2 cmul(double2 a, double2 b){ return make_double2(a.x*b.x - a.y*b.y, a.x*b.y + a.y*b.x); }
+// Every multiply-add is spelled out (here and in fa_fft_body, which keeps the compiler from forming
+// others), so that the single-chain and the batch kernel round alike.
+__device__ __forceinline__ double2 cmul(double2 a, double2 b)
+{
+#pragma clang fp contract(off)
+	return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
+}
 __device__ __forceinline__ double2 cadd(double2 a, double2 b){ return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ double2 csub(double2 a, double2 b){ return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ double2 conjg(double2 a){ return make_double2(a.x, -a.y); }
@@ -55,17 +64,29 @@ __device__ __forceinline__ unsigned mode_pos(unsigned n, const FftArgs &a)
 
 __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 {
+#pragma clang fp contract(off)
 	extern __shared__ __align__(16) unsigned char smem_raw[];
 	const unsigned nt = a.nt;
 	double2 *z = reinterpret_cast<double2 *>(smem_raw);            // [nt][LW]
 	double2 *z2 = z + (size_t)nt * FFT_LW;                         // second buffer (direct sums)
 	double2 *tw = z2 + (a.pow2 ? 0 : (size_t)nt * FFT_LW);         // [nt]
+	double *gain = reinterpret_cast<double *>(tw + nt);            // [nt] (pow2): factor of each mode
 	__shared__ double red[FFT_BT];
 	const int tid = threadIdx.x;
 	const unsigned pairs = (a.mode == FFT_EVOLVE) ? 1 : 2;         // real series per complex slot
 	const unsigned l0 = bx * FFT_LW * pairs;
 
-	for(unsigned j = tid; j < nt; j += FFT_BT) tw[j] = make_double2(a.twid[2 * j], a.twid[2 * j + 1]);
+	// factor of mode n: for the transform by stages in LDS, computed where the loads below cover the square
+	// roots and divisions; the direct sums, which take far longer, leave no LDS for it at large nt
+	auto factor = [&](unsigned n){
+		const double f = a.f2[n];
+		if(a.mode == FFT_FILTER) return a.gain == 0 ? sqrt(f) / nt : (a.gain == 1 ? 1.0 / (sqrt(f) * nt) : a.h / (f * nt));
+		return a.mode == FFT_EVOLVE ? a.s / f : 2.0 * nt * f;
+	};
+	for(unsigned j = tid; j < nt; j += FFT_BT){
+		tw[j] = make_double2(a.twid[2 * j], a.twid[2 * j + 1]);
+		if(a.pow2) gain[j] = factor(j);
+	}
 	// ---- load
 	for(unsigned e = tid; e < nt * FFT_LW; e += FFT_BT){
 		const unsigned t = e / FFT_LW, l = e % FFT_LW;
@@ -76,7 +97,7 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 				const size_t q = (size_t)t * a.loc + link;
 				re = a.in0[q];
 				im = a.in1[q];
-				if(a.kickF) im += a.kick * a.kickF[q];
+				if(a.kickF) im = fma(a.kick, a.kickF[q], im);
 			}
 		}else{
 			const unsigned la = l0 + l, lb = l0 + FFT_LW + l;
@@ -90,15 +111,32 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 	// ---- forward transform
 	double2 *Z = z;
 	if(a.pow2){
-		for(unsigned half = nt >> 1; half >= 1; half >>= 1){
-			const unsigned stride = nt / (2 * half);
-			for(unsigned q = tid; q < (nt / 2) * FFT_LW; q += FFT_BT){
-				const unsigned l = q % FFT_LW, b = q / FFT_LW;
-				const unsigned grp = b / half, pos = b - grp * half;
-				const unsigned i = grp * 2 * half + pos, j = i + half;
-				const double2 u = z[(size_t)i * FFT_LW + l], v = z[(size_t)j * FFT_LW + l];
-				z[(size_t)i * FFT_LW + l] = cadd(u, v);
-				z[(size_t)j * FFT_LW + l] = cmul(csub(u, v), tw[pos * stride]);
+		// two radix-2 stages at a time on four values in registers (halves H and H / 2, H = 2^h), so
+		// half the passes through LDS and half the barriers; a last single stage when there are an
+		// odd number.  The same operations as stage by stage.
+		int h = (int)a.logn - 1;
+		for(; h >= 1; h -= 2){
+			const unsigned H = 1u << h, Q = H >> 1, sh = a.logn - 1 - h;
+			for(unsigned e = tid; e < (nt / 4) * FFT_LW; e += FFT_BT){
+				const unsigned l = e % FFT_LW, b = e / FFT_LW, pos = b & (Q - 1);
+				double2 *p = z + (size_t)(((b >> (h - 1)) << (h + 1)) + pos) * FFT_LW + l;
+				const double2 a0 = p[0], a1 = p[(size_t)Q * FFT_LW], a2 = p[(size_t)H * FFT_LW], a3 = p[(size_t)(H + Q) * FFT_LW];
+				const double2 w2 = tw[pos << (sh + 1)];
+				const double2 s0 = cadd(a0, a2), s1 = cadd(a1, a3);
+				const double2 s2 = cmul(csub(a0, a2), tw[pos << sh]), s3 = cmul(csub(a1, a3), tw[(pos + Q) << sh]);
+				p[0] = cadd(s0, s1);
+				p[(size_t)Q * FFT_LW] = cmul(csub(s0, s1), w2);
+				p[(size_t)H * FFT_LW] = cadd(s2, s3);
+				p[(size_t)(H + Q) * FFT_LW] = cmul(csub(s2, s3), w2);
+			}
+			__syncthreads();
+		}
+		if(h == 0){
+			for(unsigned e = tid; e < (nt / 2) * FFT_LW; e += FFT_BT){
+				double2 *p = z + (size_t)(e / FFT_LW) * 2 * FFT_LW + e % FFT_LW;
+				const double2 u = p[0], v = p[FFT_LW];
+				p[0] = cadd(u, v);
+				p[FFT_LW] = cmul(csub(u, v), tw[0]);
 			}
 			__syncthreads();
 		}
@@ -106,7 +144,12 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 		for(unsigned q = tid; q < nt * FFT_LW; q += FFT_BT){
 			const unsigned l = q % FFT_LW, k = q / FFT_LW;
 			double2 acc = make_double2(0, 0);
-			for(unsigned t = 0; t < nt; t++) acc = cadd(acc, cmul(z[(size_t)t * FFT_LW + l], tw[((size_t)k * t) % nt]));
+			unsigned kt = 0;                                       // k t modulo nt
+			for(unsigned t = 0; t < nt; t++){
+				acc = cadd(acc, cmul(z[(size_t)t * FFT_LW + l], tw[kt]));
+				kt += k;
+				kt = kt >= nt ? kt - nt : kt;
+			}
 			z2[(size_t)k * FFT_LW + l] = acc;
 		}
 		__syncthreads();
@@ -119,7 +162,7 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 		for(unsigned q = tid; q < nt * FFT_LW; q += FFT_BT){
 			const unsigned l = q % FFT_LW, n = q / FFT_LW;
 			const double2 v = Z[(size_t)mode_pos(n, a) * FFT_LW + l];
-			e += (v.x * v.x + v.y * v.y) / (2.0 * nt * a.f2[n]);
+			e += fma(v.x, v.x, v.y * v.y) / (a.pow2 ? gain[n] : factor(n));
 		}
 		red[tid] = e;
 		__syncthreads();
@@ -133,8 +176,7 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 	if(a.mode == FFT_FILTER){
 		for(unsigned q = tid; q < nt * FFT_LW; q += FFT_BT){
 			const unsigned l = q % FFT_LW, n = q / FFT_LW;
-			const double f = a.f2[n];
-			const double g = a.gain == 0 ? sqrt(f) / nt : (a.gain == 1 ? 1.0 / (sqrt(f) * nt) : a.h / (f * nt));
+			const double g = a.pow2 ? gain[n] : factor(n);
 			double2 &v = Z[(size_t)mode_pos(n, a) * FFT_LW + l];
 			v = make_double2(g * v.x, g * v.y);
 		}
@@ -146,9 +188,9 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 			const double2 zn = Z[(size_t)pn * FFT_LW + l], zm = conjg(Z[(size_t)pm * FFT_LW + l]);
 			const double2 X = make_double2(0.5 * (zn.x + zm.x), 0.5 * (zn.y + zm.y));
 			const double2 P = make_double2(0.5 * (zn.y - zm.y), -0.5 * (zn.x - zm.x));   // (zn - zm)/(2i)
-			const double f = a.f2[n], sw = a.s * f, s1w = a.s / f;
-			const double2 Xn = make_double2(a.c * X.x + s1w * P.x, a.c * X.y + s1w * P.y);
-			const double2 Pn = make_double2(a.c * P.x - sw * X.x, a.c * P.y - sw * X.y);
+			const double sw = a.s * a.f2[n], s1w = a.pow2 ? gain[n] : factor(n);
+			const double2 Xn = make_double2(fma(a.c, X.x, s1w * P.x), fma(a.c, X.y, s1w * P.y));
+			const double2 Pn = make_double2(fma(a.c, P.x, -(sw * X.x)), fma(a.c, P.y, -(sw * X.y)));
 			// Z'_n = X' + i P',  Z'_-n = conj X' + i conj P'
 			Z[(size_t)pn * FFT_LW + l] = make_double2(Xn.x - Pn.y, Xn.y + Pn.x);
 			if(m != n) Z[(size_t)pm * FFT_LW + l] = make_double2(Xn.x + Pn.y, -Xn.y + Pn.x);
@@ -158,16 +200,32 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 
 	// ---- inverse transform (unnormalised; the 1/nt is in the per-mode factors)
 	if(a.pow2){
-		for(unsigned half = 1; half <= nt / 2; half <<= 1){
-			const unsigned stride = nt / (2 * half);
-			for(unsigned q = tid; q < (nt / 2) * FFT_LW; q += FFT_BT){
-				const unsigned l = q % FFT_LW, b = q / FFT_LW;
-				const unsigned grp = b / half, pos = b - grp * half;
-				const unsigned i = grp * 2 * half + pos, j = i + half;
-				const double2 u = z[(size_t)i * FFT_LW + l];
-				const double2 v = cmul(z[(size_t)j * FFT_LW + l], conjg(tw[pos * stride]));
-				z[(size_t)i * FFT_LW + l] = cadd(u, v);
-				z[(size_t)j * FFT_LW + l] = csub(u, v);
+		// halves Q = 2^h and H = 2 Q at a time, after a first single stage when there are an odd number
+		unsigned h = 0;
+		if(a.logn & 1){
+			for(unsigned e = tid; e < (nt / 2) * FFT_LW; e += FFT_BT){
+				double2 *p = z + (size_t)(e / FFT_LW) * 2 * FFT_LW + e % FFT_LW;
+				const double2 u = p[0], v = cmul(p[FFT_LW], conjg(tw[0]));
+				p[0] = cadd(u, v);
+				p[FFT_LW] = csub(u, v);
+			}
+			__syncthreads();
+			h = 1;
+		}
+		for(; h + 1 < a.logn; h += 2){
+			const unsigned Q = 1u << h, H = Q << 1, sh = a.logn - 2 - h;      // H's twiddles: pos << sh
+			for(unsigned e = tid; e < (nt / 4) * FFT_LW; e += FFT_BT){
+				const unsigned l = e % FFT_LW, b = e / FFT_LW, pos = b & (Q - 1);
+				double2 *p = z + (size_t)(((b >> h) << (h + 2)) + pos) * FFT_LW + l;
+				const double2 w1 = conjg(tw[pos << (sh + 1)]);
+				const double2 a0 = p[0], a1 = cmul(p[(size_t)Q * FFT_LW], w1), a2 = p[(size_t)H * FFT_LW],
+					a3 = cmul(p[(size_t)(H + Q) * FFT_LW], w1);
+				const double2 s0 = cadd(a0, a1), s1 = csub(a0, a1), s2 = cmul(cadd(a2, a3), conjg(tw[pos << sh])),
+					s3 = cmul(csub(a2, a3), conjg(tw[(pos + Q) << sh]));
+				p[0] = cadd(s0, s2);
+				p[(size_t)Q * FFT_LW] = cadd(s1, s3);
+				p[(size_t)H * FFT_LW] = csub(s0, s2);
+				p[(size_t)(H + Q) * FFT_LW] = csub(s1, s3);
 			}
 			__syncthreads();
 		}
@@ -175,7 +233,12 @@ __device__ __forceinline__ void fa_fft_body(const FftArgs &a, unsigned bx)
 		for(unsigned q = tid; q < nt * FFT_LW; q += FFT_BT){
 			const unsigned l = q % FFT_LW, t = q / FFT_LW;
 			double2 acc = make_double2(0, 0);
-			for(unsigned k = 0; k < nt; k++) acc = cadd(acc, cmul(z2[(size_t)k * FFT_LW + l], conjg(tw[((size_t)k * t) % nt])));
+			unsigned kt = 0;
+			for(unsigned k = 0; k < nt; k++){
+				acc = cadd(acc, cmul(z2[(size_t)k * FFT_LW + l], conjg(tw[kt])));
+				kt += t;
+				kt = kt >= nt ? kt - nt : kt;
+			}
 			z[(size_t)t * FFT_LW + l] = acc;
 		}
 		__syncthreads();
@@ -243,7 +306,7 @@ static int fft_shape(ephmc_ctx *c, const FftArgs &a, unsigned *blocks, size_t *l
 {
 	const unsigned per = (a.mode == FFT_EVOLVE) ? FFT_LW : 2 * FFT_LW;
 	*blocks = (c->loc + per - 1) / per;
-	*lds = (size_t)c->nt * FFT_LW * sizeof(double2) * (a.pow2 ? 1 : 2) + (size_t)c->nt * sizeof(double2);
+	*lds = (size_t)c->nt * FFT_LW * sizeof(double2) * (a.pow2 ? 1 : 2) + (size_t)c->nt * (sizeof(double2) + (a.pow2 ? sizeof(double) : 0));
 	if(*lds > 160 * 1024){ set_error("fft: nt = %u needs %zu B of LDS", c->nt, *lds); return EPHMC_ERR_UNSUPPORTED; }
 	return EPHMC_OK;
 }

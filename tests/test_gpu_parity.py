@@ -314,6 +314,31 @@ def test_force_ragged(monkeypatch, l1, l2, nt, cols, precision, tol, checkpoint)
     assert rel(Fg, Fo) < tol
 
 
+# every number of stages (odd: one single stage), the largest transforms that LDS holds, direct sums
+@pytest.mark.parametrize("nt", [1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 1024, 3, 95, 590])
+def test_boson_transforms_vs_numpy(nt):
+    """Free-boson draw, momentum refresh, kinetic energy and exact flow against numpy's transforms; the
+    direct sums add nt terms, so their rounding is nt eps at most."""
+    say("boson transforms, nt =", nt)
+    om = OracleModel(3, 1, nt)
+    ctx = gpu_context(om)
+    rng = np.random.default_rng(nt)
+    n1, n2 = rng.standard_normal((2, nt, 9))
+    f2 = om.omega + (2 * np.sin(np.pi * np.arange(nt // 2 + 1) / nt)) ** 2 / om.omega
+
+    def scaled(a, g):
+        return np.fft.irfft(np.fft.rfft(a, axis=0) * g[:, None], n=nt, axis=0) if nt > 1 else a * g[0]
+
+    tol = 1e-13 * max(1, nt / 64) * max(1.0, (f2.max() / f2.min()) ** 0.5 * 1e-2)
+    x, p = scaled(n1, f2 ** -.5), scaled(n2, f2 ** .5)
+    assert rel(ctx.sample_free_bosons(n1.ravel()), x.ravel()) < tol
+    assert rel(ctx.sample_fourier_momenta(n2.ravel()), p.ravel()) < tol
+    assert ctx.energy_momenta(p.ravel()) == pytest.approx(.5 * (n2 ** 2).sum(), rel=1e-11)
+    gx, gp = ctx.evolve_bosons(x.ravel(), p.ravel(), 0.3)
+    assert rel(gx, (np.cos(.3) * x + np.sin(.3) * scaled(p, 1 / f2)).ravel()) < 10 * tol
+    assert rel(gp, (np.cos(.3) * p - np.sin(.3) * scaled(x, f2)).ravel()) < 10 * tol
+
+
 @pytest.mark.parametrize("nt", [1, 2, 8, 12, 32, 48])
 def test_boson_kernels(nt):
     say("bosons", nt)
