@@ -152,6 +152,29 @@ def test_logdet_inverse_diagonally_dominant_no_fallback():
     assert ctx.gj_fallbacks() == 0
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 15, 17, 31, 33, 47, 52, 63, 64, 65, 67, 95, 96, 97, 129, 160, 191, 1023, 1400, 1401, 1409, 1472, 1531])
+def test_logdet_inverse_sizes(n):
+    """Every form of the inversion at the edges of its range (one workgroup to N = 64, blocks of 32
+    columns, blocks of 64 above N = 1400) and at last blocks of every kind: diagonally dominant with
+    pivots of both signs, so that the fast path serves it, and the same matrix with one entry that
+    asks for a row exchange late in it, so that the pivoted one does.  The condition numbers are of
+    order 10 and numpy's own inverse is the reference: 1e-12 covers n eps kappa of both."""
+    ctx = gpu_context(OracleModel(n, 1, 1))
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n)) * (0.3 / np.sqrt(n)) + np.diag(np.where(rng.random(n) < 0.3, -2.0, 2.0))
+    for exchange in (False, True):
+        if exchange:
+            if n == 1:
+                break
+            A[n - 1, n - 2] = 6.0
+        say("gj sizes", n, exchange)
+        ld, sg, inv = ctx.logdet_inv(A.T.copy().ravel())
+        s0, l0 = np.linalg.slogdet(A)
+        assert ctx.gj_fallbacks() == int(exchange)
+        assert ld == pytest.approx(l0, rel=1e-12) and sg == int(s0)
+        assert rel(inv.reshape(n, n).T, np.linalg.inv(A)) < 1e-12
+
+
 @pytest.mark.parametrize("l1,l2,nt", [(6, 6, 32), (16, 16, 64)])
 def test_logdet_inverse_M_hat(l1, l2, nt):
     say("gj M_hat", l1, l2, nt)
