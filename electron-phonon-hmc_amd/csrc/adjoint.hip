@@ -16,7 +16,18 @@
 // Sweep: tau = nt-1 ... 0 with W_{nt-1} = M_hat^{-1}, W_{tau-1} = B_tau W_tau = sum_n c_n W_n.
 // T_tau comes from checkpoints T_{s k} stored by the forward chain every k slices and is
 // recomputed inside the segment (stored to a workgroup-private scratch, then read backwards).
+//
+// S by Horner, S_{deg-1} = c_deg T, S_a = c_{a+1} T + A S_{a+1}: one multiply-add per stencil where the
+// sum over the powers of T takes deg - b of them in step b, and only S itself is held.  A slice is a row
+// of phases (write a vector to LDS, barrier, read the neighbours), deg - 1 for S and deg for W.  At up to
+// 256 sites (512 in fp64) their latency bounds the sweep, so the next slice's S is built under this
+// slice's W phases: deg barriers a slice instead of 2 deg - 1, 32 slices of 6x6 38.5 -> 34.9 us, 64 of
+// 16x16 56.4 -> 45.4.  With 1024 threads registers are what is short: 32 slices of 32x32 in fp64 at four
+// columns 340 -> 262 us, of 36x36 at two 1721 -> 1209 (no more spills in the loop), in fp32 134 -> 128; there a
+// workgroup's reads of LDS take 4.5 of the 8 us per slice in fp64, 2.2 of 4 in fp32, and T and the partial sums
+// about as long at the rate of memory.
 #include "internal.h"
+#include <type_traits>
 
 namespace ephmc {
 
@@ -109,12 +120,6 @@ __device__ void reduce_links(const P *__restrict__ part, unsigned nwg, unsigned 
 	}
 }
 
-// A site's C values fit one 16-byte LDS read (fp32 up to 4 columns, fp64 up to 2): with one site
-// per thread the register footprint allows the lean form of the sweep (all lanes active, six
-// neighbour reads issued together, constant LDS offsets)
-template <typename R, int C>
-constexpr bool adj_lean(){ return C * sizeof(R) <= 16; }
-
 // Place of value (site, c) in an LDS buffer of np sites: the C columns in planes of the widest read
 // (16 bytes), each [site][column].  One plane up to 16 bytes per site; fp64 at 4 columns takes two: a
 // 32-byte stride between sites would put lanes 8 apart on the same banks in every read.
@@ -128,38 +133,32 @@ __device__ __forceinline__ size_t adj_at(unsigned site, int c, unsigned np)
 	return V == C ? (size_t)site * C + c : (size_t)(c / V) * np * V + (size_t)site * V + c % V;
 }
 
-// BATCH: the six neighbour reads are issued before any of them is used; otherwise each is read
-// just before its sums, which holds fewer registers. The sum is taken in the order d = 0..5
-// either way.
-template <typename R, int C, bool BATCH>
+// The neighbours are read NB at a time (6: all before any is used, 1: each just before its sums), which
+// sets how many registers hold them.  The sum is taken in the order d = 0..5 either way.
+template <typename R, int C, int NB>
 __device__ __forceinline__ void gather6(const R *__restrict__ buf, unsigned np, const int (&nbr)[6], const R (&cf)[6], R mu,
 		const R (&own)[C], R (&out)[C])
 {
 #pragma unroll
 	for(int c = 0; c < C; c++) out[c] = mu * own[c];
-	if constexpr(BATCH){
-		R nv[6][C];
 #pragma unroll
-		for(int d = 0; d < 6; d++)
+	for(int d0 = 0; d0 < 6; d0 += NB){
+		R nv[NB][C];
 #pragma unroll
-			for(int c = 0; c < C; c++) nv[d][c] = buf[adj_at<R, C>(nbr[d], c, np)];
+		for(int d = 0; d < NB; d++)
 #pragma unroll
-		for(int d = 0; d < 6; d++)
+			for(int c = 0; c < C; c++) nv[d][c] = buf[adj_at<R, C>(nbr[d0 + d], c, np)];
 #pragma unroll
-			for(int c = 0; c < C; c++) out[c] = fmac(cf[d], nv[d][c], out[c]);
-	}else{
+		for(int d = 0; d < NB; d++)
 #pragma unroll
-		for(int d = 0; d < 6; d++){
-#pragma unroll
-			for(int c = 0; c < C; c++) out[c] = fmac(cf[d], buf[adj_at<R, C>(nbr[d], c, np)], out[c]);
-		}
+			for(int c = 0; c < C; c++) out[c] = fmac(cf[d0 + d], nv[d][c], out[c]);
 	}
 }
 
 template <typename R, int C, int BT, int S>
 __host__ __device__ constexpr size_t adj_buf_stride(unsigned ns)
 {
-	return (sizeof(R) == 4 || (adj_lean<R, C>() && S == 1)) ? (size_t)C * BT * S : (size_t)C * ns;
+	return (sizeof(R) == 4 || S == 1) ? (size_t)C * BT * S : (size_t)C * ns;
 }
 
 template <typename R, int C, int BT, int S>
@@ -175,16 +174,24 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 {
 	extern __shared__ __align__(16) unsigned char smem_raw[];
 	const unsigned ns = a.ns;
-	// lean one-site form (fp64 only up to degree 4; beyond it, with two sites per thread, or in
-	// fp64 at 4 columns, the guarded form and the run-time degree hold fewer registers); fp32
-	// always reads the six neighbours together
-	constexpr bool LEAN = adj_lean<R, C>() && S == 1 && (sizeof(R) == 4 || DEG <= 4);
-	constexpr bool BATCH = sizeof(R) == 4 || LEAN;
+	// neighbours read together: all six where the registers allow it
+	constexpr int NB = sizeof(R) == 4 || (S == 1 && C <= 2 && DEG <= 4) ? 6 : 1;
+	// with one site per thread every lane loads and gathers, so no lane needs zero values of its own
+	constexpr bool ALL_LANES = S == 1;
+	// the next slice's S built under this slice's W phases (above these sizes its registers cost more than
+	// the barriers: fp32 at 21x19 61.7 us per 32 slices against 65.0)
+	constexpr bool MERGE = S == 1 && (BT <= 256 || (BT <= 512 && sizeof(R) == 8));
+	constexpr bool TIGHT = sizeof(R) == 8 && C == 4;
+	// the phase that loads ahead: the first, or, where registers are short, one that S_0, S_1 have left
+	constexpr int PRE = TIGHT ? 2 % DEG : 0;
+	// two sites per thread in fp64 have no registers to load ahead
+	constexpr bool AHEAD = S == 1 || sizeof(R) == 4;
 	// LDS: buf0, buf1, wb0, wb1 of bs values each, then hx [site][3] and the reduction scratch; in
-	// fp32 and in the lean fp64 form bs is the constant C * BT * S, so the four buffers sit at
+	// fp32 and with one site per thread bs is the constant C * BT * S, so the four buffers sit at
 	// fixed offsets from one neighbour address and a read needs no address add (the offsets fit
 	// the 16-bit immediate when C * BT * S * sizeof(R) <= 16 KiB)
 	const size_t bs = adj_buf_stride<R, C, BT, S>(ns);
+	const unsigned pl = (unsigned)(bs / C);     // sites of a plane
 	R *buf0 = reinterpret_cast<R *>(smem_raw);
 	R *buf1 = buf0 + bs;
 	R *wb0 = buf0 + 2 * bs;
@@ -241,23 +248,23 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 				for(int j = 0; j < S; j++)
 					if(act[j])
 #pragma unroll
-						for(int c = 0; c < C; c++) buf0[adj_at<R, C>(site[j], c, ns)] = v[j][c];
+						for(int c = 0; c < C; c++) buf0[adj_at<R, C>(site[j], c, pl)] = v[j][c];
 				__syncthreads();
 #pragma unroll
 				for(int j = 0; j < S; j++)
-					if(act[j]) gather6<R, C, BATCH>(buf0, ns, nbr[j], cf[j], a.mu, v[j], w[j]);
+					if(act[j]) gather6<R, C, NB>(buf0, pl, nbr[j], cf[j], a.mu, v[j], w[j]);
 				if(a.cplx[p]){
 #pragma unroll
 					for(int j = 0; j < S; j++)
 						if(act[j])
 #pragma unroll
-							for(int c = 0; c < C; c++) buf1[adj_at<R, C>(site[j], c, ns)] = w[j][c];
+							for(int c = 0; c < C; c++) buf1[adj_at<R, C>(site[j], c, pl)] = w[j][c];
 					__syncthreads();
 #pragma unroll
 					for(int j = 0; j < S; j++){
 						if(!act[j]) continue;
 						R z[C];
-						gather6<R, C, BATCH>(buf1, ns, nbr[j], cf[j], a.mu, w[j], z);
+						gather6<R, C, NB>(buf1, pl, nbr[j], cf[j], a.mu, w[j], z);
 #pragma unroll
 						for(int c = 0; c < C; c++) v[j][c] = v[j][c] + fmac(a.a_quad[p], z[c], a.a_lin[p] * w[j][c]);
 					}
@@ -287,41 +294,35 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 			wv[j][c] = val;
 		}
 
-	// lean form: every lane loads and gathers, so no lane needs zero values of its own, and the
-	// degree is the constant DEG
-	constexpr bool ALL_LANES = LEAN;
-	const int deg = ALL_LANES ? DEG : a.deg;
-	// coefficients and T of slice tau-1 are loaded while slice tau is processed (each thread
-	// reads back only the scratch entries it wrote itself)
-	R cfn[S][6], tn0[S][C];
-	auto load_slice = [&](int tau){
+	auto load_cf = [&](int tau, R (&f)[S][6]){
 		const R *cft = a.coef + (size_t)tau * 6 * ns;
+#pragma unroll
+		for(int j = 0; j < S; j++)
+#pragma unroll
+			for(int d = 0; d < 6; d++){
+				// (a lane past the last site reads site ns-1 and stores nothing)
+				if constexpr(ALL_LANES) f[j][d] = (cft + d * ns)[act[j] ? site[j] : ns - 1];
+				else f[j][d] = act[j] ? cft[d * ns + site[j]] : (R)0;
+			}
+	};
+	auto load_t = [&](int tau, R (&t)[S][C]){
 		const R *tsrc = a.direct ? a.ck + (size_t)(tau - a.tau_b) * ns * ns + (size_t)col0 * ns
 		                         : seg + (size_t)(tau - a.tau_b) * C * ns;
 #pragma unroll
-		for(int j = 0; j < S; j++){
-			if constexpr(ALL_LANES){
-				// A lane past the last site reads site ns-1 and stores nothing. A column past the
-				// last (last workgroup only) reads column ns-1; its W column is zero throughout the
-				// sweep, so its products add zeros to the bond sums.
-				const unsigned sl = act[j] ? site[j] : ns - 1;
+		for(int j = 0; j < S; j++)
 #pragma unroll
-				for(int d = 0; d < 6; d++) cfn[j][d] = cft[d * ns + sl];
-#pragma unroll
-				for(int c = 0; c < C; c++) tn0[j][c] = tsrc[(size_t)(colok(c) ? c : ns - 1 - col0) * ns + sl];
-			}else{
-#pragma unroll
-				for(int d = 0; d < 6; d++) cfn[j][d] = act[j] ? cft[d * ns + site[j]] : (R)0;
-#pragma unroll
-				for(int c = 0; c < C; c++) tn0[j][c] = (act[j] && colok(c)) ? tsrc[(size_t)c * ns + site[j]] : (R)0;
+			for(int c = 0; c < C; c++){
+				// A column past the last (last workgroup only) reads column ns-1; its W column is zero
+				// throughout the sweep, so its products add zeros to the bond sums.
+				if constexpr(ALL_LANES) t[j][c] = (tsrc + (size_t)(colok(c) ? c : ns - 1 - col0) * ns)[act[j] ? site[j] : ns - 1];
+				else t[j][c] = (act[j] && colok(c)) ? tsrc[(size_t)c * ns + site[j]] : (R)0;
 			}
-		}
 	};
 	// bond(i, 2k) = H[i][2k] + H[nb(i,2k)][2k+1]: the H[.][2k+1] of a slice go to LDS (hx) at
-	// its end and, in FP32, the bond sums are written after the next slice's first barrier
-	// (after the last slice, after one more barrier); FP64 keeps a barrier of its own per slice,
-	// as holding H[.][2k] across the slice would spill registers
-	constexpr bool FOLD = sizeof(R) == 4;
+	// its end and, with FOLD, the bond sums are written after the next slice's first barrier
+	// (after the last slice, after one more barrier); fp64 at 4 columns keeps a barrier of its own per
+	// slice, as holding H[.][2k] across the slice would spill registers
+	constexpr bool FOLD = sizeof(R) == 4 || C <= 2;
 	R hb[S][3];
 	int tau_out = -1;
 	auto flush_bonds = [&](){
@@ -332,128 +333,136 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 #pragma unroll
 				for(int k = 0; k < 3; k++) out[(size_t)site[j] * 3 + k] = hb[j][k] + hx[(size_t)nbr[j][2 * k] * 3 + k];
 	};
-	// W_0 of a slice goes to wbs[0] as soon as it is known (here, then at the end of each slice);
-	// the T-power barriers make it visible, so the first W phase needs no barrier of its own
-	auto put_w0 = [&](){
+	auto put = [&](R *b, const R (&v)[S][C]){
 #pragma unroll
 		for(int j = 0; j < S; j++)
 			if(act[j])
 #pragma unroll
-				for(int c = 0; c < C; c++) wbs[0][adj_at<R, C>(site[j], c, ns)] = wv[j][c];
+				for(int c = 0; c < C; c++) b[adj_at<R, C>(site[j], c, pl)] = v[j][c];
 	};
-	if(a.w0_early) put_w0();
-	load_slice(a.tau_e - 1);
-	for(int tau = a.tau_e - 1; tau >= a.tau_b; tau--){
-		R t[S][C];
+	R *const sbs[2] = {buf0, buf1};
+	// S_q in sa[q] (even slices of the sweep) or sa[DEG - 2 - q] (odd ones; S_{DEG-1} always in the last): the
+	// slots that a slice's S leave, in the order q = 0 .. DEG - 2, take the next slice's DEG - 2 .. 0
+	R sa[DEG][S][C], t[S][C], cfn[S][6];
+	// S_q = c_{q+1} T + A S_{q+1} for the S_{q+1} in b
+	auto next_s = [&](int q, const R *b, const R (&f)[S][6], const R (&sq1)[S][C], R (&sq)[S][C]){
 #pragma unroll
 		for(int j = 0; j < S; j++){
+			R sn[C];
+			if(ALL_LANES || act[j]) gather6<R, C, NB>(b, pl, nbr[j], f[j], a.mu, sq1[j], sn);
+			else
 #pragma unroll
-			for(int d = 0; d < 6; d++) cf[j][d] = cfn[j][d];
+				for(int c = 0; c < C; c++) sn[c] = 0;
 #pragma unroll
-			for(int c = 0; c < C; c++) t[j][c] = tn0[j][c];
+			for(int c = 0; c < C; c++) sq[j][c] = fmac(a.cm[q + 1], t[j][c], sn[c]);
 		}
-		if(tau > a.tau_b) load_slice(tau - 1);
-
-		// S_a = sum_b c_{a+b+1} T_b, built while the powers T_b = A^b T are formed
-		R sa[DEG][S][C];
+	};
+	auto scaled_t = [&](R (&v)[S][C]){
 #pragma unroll
-		for(int q = 0; q < DEG; q++)
+		for(int j = 0; j < S; j++)
 #pragma unroll
-			for(int j = 0; j < S; j++)
+			for(int c = 0; c < C; c++) v[j][c] = a.cm[DEG] * t[j][c];
+	};
+	// a slice's S by itself
+	auto build_s = [&](){
+		scaled_t(sa[DEG - 1]);
 #pragma unroll
-				for(int c = 0; c < C; c++) sa[q][j][c] = (q < deg) ? a.cm[q + 1] * t[j][c] : (R)0;
-		// unrolled: b is a constant, so bb is a known LDS buffer
-#pragma unroll
-		for(int b = 1; b < DEG; b++){
-			if(b >= deg) break;
-			R *bb = ((b - 1) & 1) ? buf1 : buf0;
-#pragma unroll
-			for(int j = 0; j < S; j++)
-				if(act[j])
-#pragma unroll
-					for(int c = 0; c < C; c++) bb[adj_at<R, C>(site[j], c, ns)] = t[j][c];
+		for(int q = DEG - 2; q >= 0; q--){
+			// (the last one, q = 0, leaves buf0 to the phase that follows it without a barrier)
+			put(sbs[(q & 1) ^ 1], sa[q + 1]);
 			__syncthreads();
-			if(FOLD && a.w0_early && b == 1 && tau_out >= 0) flush_bonds();
-#pragma unroll
-			for(int j = 0; j < S; j++){
-				// with ALL_LANES a thread past the last site gathers too (neighbour 0, in bounds)
-				// and stores nothing
-				R tn[C];
-				if(ALL_LANES || act[j]) gather6<R, C, BATCH>(bb, ns, nbr[j], cf[j], a.mu, t[j], tn);
-				else
-#pragma unroll
-					for(int c = 0; c < C; c++) tn[c] = 0;
-#pragma unroll
-				for(int c = 0; c < C; c++) t[j][c] = tn[c];
-			}
-#pragma unroll
-			for(int q = 0; q < DEG; q++)
-				if(q + b < deg)
-#pragma unroll
-					for(int j = 0; j < S; j++)
-#pragma unroll
-						for(int c = 0; c < C; c++) sa[q][j][c] = fmac(a.cm[q + b + 1], t[j][c], sa[q][j][c]);
+			if(FOLD && a.w0_early && q == DEG - 2 && tau_out >= 0) flush_bonds();
+			next_s(q, sbs[(q & 1) ^ 1], cf, sa[q + 1], sa[q]);
 		}
-
+	};
+	if(AHEAD){
+		load_cf(a.tau_e - 1, cf);
+		load_t(a.tau_e - 1, t);
+	}
+	if(a.w0_early) put(wbs[0], wv);
+	if constexpr(MERGE){
+		build_s();
+		load_cf(max(a.tau_e - 2, a.tau_b), cfn);
+		load_t(max(a.tau_e - 2, a.tau_b), t);
+	}
+	// coefficients and T of a later slice, loaded while this one is processed (past the segment's first slice:
+	// that one again, not used)
+	R cfl[S][6], tl[S][C];
+	auto load_next = [&](int tau){
+		load_cf(max(tau - 1 - MERGE, a.tau_b), cfl);
+		load_t(max(tau - 1 - MERGE, a.tau_b), tl);
+	};
+	auto slice = [&](int tau, auto odd, auto more_){
+		constexpr bool ODD = decltype(odd)::value, more = decltype(more_)::value;
 		// W powers with the half-bond sums taken from the same neighbour reads:
 		// H[i][d] = sum_{q,c} S_q[i,c] W_q[nb(i,d),c]
-		R h[S][6];
-		R acc[S][C], wa[S][C];
+		R h[S][6], acc[S][C], wa[S][C];
+		constexpr auto slot = [](int i){ return ODD && i < DEG - 1 ? DEG - 2 - i : i; };
+		// a phase's sums end before the next one's barrier, under its writes to LDS, or, where registers are
+		// short, before those: the compiler would sink them
+		// to their use at the slice's end, with every neighbour's values kept in registers (fp32, 4 columns:
+		// 234 of them instead of 90)
+		auto settle = [&](int q){
 #pragma unroll
-		for(int j = 0; j < S; j++){
+			for(int j = 0; j < S; j++){
+				if(S == 1 || sizeof(R) == 4)
 #pragma unroll
-			for(int d = 0; d < 6; d++) h[j][d] = 0;
+					for(int d = 0; d < 6; d++) asm volatile("" : "+v"(h[j][d]));
+				if(MERGE || (sizeof(R) == 8 && S == 1))
+#pragma unroll
+					for(int c = 0; c < C; c++) asm volatile("" : "+v"(acc[j][c]), "+v"(wa[j][c]), "+v"(sa[slot(q)][j][c]));
+			}
+		};
+#pragma unroll
+		for(int j = 0; j < S; j++)
 #pragma unroll
 			for(int c = 0; c < C; c++){
 				acc[j][c] = a.cm[0] * wv[j][c];
 				wa[j][c] = wv[j][c];
 			}
-		}
 #pragma unroll
 		for(int q = 0; q < DEG; q++){
-			if(q >= deg) break;
-			R *wb = wbs[q & 1];
-			if(q > 0 || !a.w0_early){
+			R *wb = wbs[q & 1], *sb = sbs[q & 1];
+			R s1[S][C];
+			if(q > 0 || !a.w0_early) put(wb, wa);
+			if(MERGE && more && q < DEG - 1){
+				if(q == 0) scaled_t(s1);
 #pragma unroll
 				for(int j = 0; j < S; j++)
-					if(act[j])
 #pragma unroll
-						for(int c = 0; c < C; c++) wb[adj_at<R, C>(site[j], c, ns)] = wa[j][c];
-				__syncthreads();
-				if(FOLD && !a.w0_early && q == 0 && tau_out >= 0) flush_bonds();
+					for(int c = 0; c < C; c++) if(q > 0) s1[j][c] = sa[slot(q > 0 ? q - 1 : 0)][j][c];
+				put(sb, s1);
 			}
+			if(!TIGHT && q > 0) settle(q - 1);
+			// (W_0 written ahead is visible behind the barriers of S)
+			if(MERGE || q > 0 || !a.w0_early){
+				__syncthreads();
+				if(FOLD && q == 0 && tau_out >= 0) flush_bonds();
+			}
+			if(more && q == PRE) load_next(tau);
 #pragma unroll
 			for(int j = 0; j < S; j++){
-				if(!act[j]) continue;
+				if(!ALL_LANES && !act[j]) continue;
 				R wn[C];
-				// BATCH: all six neighbour reads are issued before any of them is used (otherwise
-				// each is read just before its sums; same arithmetic)
-				constexpr int NV = BATCH ? 6 : 1;
-				R nv[NV][C];
-				if constexpr(NV == 6){
-#pragma unroll
-					for(int d = 0; d < 6; d++)
-#pragma unroll
-						for(int c = 0; c < C; c++) nv[d][c] = wb[adj_at<R, C>(nbr[j][d], c, ns)];
-				}
 #pragma unroll
 				for(int c = 0; c < C; c++) wn[c] = a.mu * wa[j][c];
 #pragma unroll
-				for(int d = 0; d < 6; d++){
-					const int dv = NV == 6 ? d : 0;
-					if constexpr(NV == 1){
+				for(int d0 = 0; d0 < 6; d0 += NB){
+					R nv[NB][C];
 #pragma unroll
-						for(int c = 0; c < C; c++) nv[0][c] = wb[adj_at<R, C>(nbr[j][d], c, ns)];
-					}
-					R hs = 0;
+					for(int d = 0; d < NB; d++)
 #pragma unroll
-					for(int c = 0; c < C; c++){
-						hs = fmac(sa[q][j][c], nv[dv][c], hs);
-						wn[c] = fmac(cf[j][d], nv[dv][c], wn[c]);
+						for(int c = 0; c < C; c++) nv[d][c] = wb[adj_at<R, C>(nbr[j][d0 + d], c, pl)];
+#pragma unroll
+					for(int d = 0; d < NB; d++){
+						R hs = 0;
+#pragma unroll
+						for(int c = 0; c < C; c++){
+							hs = fmac(sa[slot(q)][j][c], nv[d][c], hs);
+							wn[c] = fmac(cf[j][d0 + d], nv[d][c], wn[c]);
+						}
+						h[j][d0 + d] = q == 0 ? hs : h[j][d0 + d] + hs;
 					}
-					// (with ALL_LANES the first phase's sum is taken as is; the guarded form adds
-					// it to zero, which holds fewer registers)
-					h[j][d] = (ALL_LANES && q == 0) ? hs : h[j][d] + hs;
 				}
 #pragma unroll
 				for(int c = 0; c < C; c++){
@@ -461,6 +470,8 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 					acc[j][c] = fmac(a.cm[q + 1], wn[c], acc[j][c]);
 				}
 			}
+			if(MERGE && more && q < DEG - 1) next_s(DEG - 2 - q, sb, cfn, s1, sa[slot(q)]);
+			if(TIGHT) settle(q);
 		}
 #pragma unroll
 		for(int j = 0; j < S; j++){
@@ -480,10 +491,40 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 		for(int j = 0; j < S; j++)
 #pragma unroll
 			for(int c = 0; c < C; c++) wv[j][c] = acc[j][c];
-		// wbs[0] was last read in W phase deg - 2 (deg is even), before the barrier of phase deg - 1
-		if(a.w0_early){
-			if((deg - 1) % 2 == 0) __syncthreads();
-			put_w0();
+		if(more){
+			if(MERGE) scaled_t(sa[DEG - 1]);
+#pragma unroll
+			for(int j = 0; j < S; j++){
+#pragma unroll
+				for(int d = 0; d < 6; d++){
+					cf[j][d] = MERGE ? cfn[j][d] : cfl[j][d];
+					cfn[j][d] = cfl[j][d];
+				}
+#pragma unroll
+				for(int c = 0; c < C; c++) t[j][c] = tl[j][c];
+			}
+		}
+		// wbs[0] was last read in phase DEG - 2 (DEG is even), before the barrier of phase DEG - 1
+		if(a.w0_early) put(wbs[0], wv);
+	};
+	int tau = a.tau_e - 1;
+	if constexpr(MERGE){
+		for(; tau > a.tau_b + 1; tau -= 2){
+			slice(tau, std::false_type{}, std::true_type{});
+			slice(tau - 1, std::true_type{}, std::true_type{});
+		}
+		if(tau > a.tau_b){
+			slice(tau, std::false_type{}, std::true_type{});
+			slice(tau - 1, std::true_type{}, std::false_type{});
+		} else slice(tau, std::false_type{}, std::false_type{});
+	} else {
+		for(; tau >= a.tau_b; tau--){
+			if(!AHEAD){
+				load_cf(tau, cf);
+				load_t(tau, t);
+			}
+			build_s();
+			slice(tau, std::false_type{}, std::bool_constant<AHEAD>{});
 		}
 	}
 	__syncthreads();

@@ -145,17 +145,20 @@ int timer_end(ephmc_ctx *c, const char *group)
 	return EPHMC_OK;
 }
 
-// Columns per workgroup of the adjoint sweep: the widest that fits LDS and keeps at least one
-// workgroup per CU (at 32x32: 4 columns, 0.13 ms per 32-slice launch in fp32 and 0.32 ms in
-// fp64).  EPHMC_ADJOINT_COLS overrides it for tuning sweeps.
+// Columns per workgroup of the adjoint sweep.  A slice's partial bond sums (3 N per workgroup) and its
+// coefficients are paid per workgroup, so wide ones win even where they leave CUs idle, until latency is
+// what counts: per 32 slices 16x16 45 us at 1 column and 53 at 2 (fp64); 21x19 110 at 1, 81 at 2, 118 at 4
+// (fp32 72, 61, 78); 24x24 235 at 2, 194 at 4 (fp32 140, 106); 32x32 334 at 2, 262 at 4 (fp32 173, 126).  Beyond
+// 1024 sites a thread holds two and registers for two columns: 36x36 in fp32 332 at 2, 560 at 4.
+// EPHMC_ADJOINT_COLS overrides it for tuning sweeps.
 static unsigned adjoint_cols_auto(unsigned ns, int prec)
 {
 	if(const char *e = getenv("EPHMC_ADJOINT_COLS")){
 		const unsigned v = (unsigned)atoi(e);
 		if(v == 1 || v == 2 || v == 4) return v;
 	}
-	for(unsigned C = 4; C > 1; C >>= 1)
-		if(adjoint_lds(ns, prec, C) <= 160 * 1024 && (ns + C - 1) / C >= 256) return C;
+	for(unsigned C = ns <= 256 ? 1 : ns <= 512 || ns > 1024 ? 2 : 4; C > 1; C >>= 1)
+		if(adjoint_lds(ns, prec, C) <= 160 * 1024) return C;
 	return 1;
 }
 

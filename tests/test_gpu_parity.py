@@ -477,3 +477,34 @@ def test_full_size_force_finite_differences():
     say("finite-difference rel err: central eps 1e-5 %.2e, Richardson (2e-2, 4e-2) %.2e" % (err5, err))
     assert err5 < 5e-5
     assert err < 1e-7
+
+
+@pytest.mark.parametrize("l1,l2,nt,order,prec", [(1, 1, 3, 4, 0), (2, 3, 1, 4, 0), (3, 5, 2, 2, 0), (16, 16, 5, 4, 0), (16, 16, 4, 6, 1),
+                                                 (17, 16, 6, 4, 0), (21, 19, 7, 4, 0), (21, 19, 5, 2, 1), (23, 22, 3, 8, 0),
+                                                 (24, 24, 4, 4, 1), (32, 32, 3, 4, 0), (33, 32, 3, 4, 0), (36, 36, 2, 6, 1)])
+def test_force_sweep_columns(l1, l2, nt, order, prec, monkeypatch):
+    """Odd and even numbers of slices, every polynomial degree and launch size: the force sweep gives the
+    oracle's force at every number of columns per workgroup, and the same bits with W_0 written ahead
+    or not and from a recomputed T.  1e-11 (fp64) and 1e-5 (fp32) as for every force here."""
+    om = OracleModel(l1, l2, nt, beta=nt * 40 / 32, taylor=order)
+    x = field(om, 9)
+    monkeypatch.setenv("EPHMC_ADJOINT_COLS", "1")
+    base = gpu_context(om, taylor_order=order)
+    _, _, Minv = base.logdet_inv(base.M_hat(x))
+    # (beyond the sizes that the oracle finishes in seconds: the fp64 sweep of one column per workgroup)
+    ref = om.force(x, Minv, 0.0) if om.ns <= 400 else base.force(x, Minv, 0.0)
+    tol = 1e-5 if prec else 1e-11
+    for cols in (1, 2, 4):
+        monkeypatch.setenv("EPHMC_ADJOINT_COLS", str(cols))
+        bits = []
+        for early, ckpt in (("0", 1), ("1", 1), ("1", 2)):
+            monkeypatch.setenv("EPHMC_ADJOINT_W0EARLY", early)
+            say("sweep", l1, l2, nt, order, prec, cols, early, ckpt)
+            ctx = gpu_context(om, precision=prec, checkpoint=ckpt, taylor_order=order)
+            try:
+                bits.append(ctx.force(x, Minv, 0.0))
+            except ephmc().EphmcError:
+                assert l1 * l2 > 1024 and not prec and cols == 4     # over the LDS, as before
+                continue
+            assert rel(bits[-1], ref) < tol
+            np.testing.assert_array_equal(bits[-1], bits[0])
