@@ -745,7 +745,7 @@ __global__ __launch_bounds__(1024) void gj_fallback_kernel(double *__restrict__ 
 
 // N <= 64: the matrix is one diagonal block, so that one workgroup inverts it in LDS, sums its pivots and,
 // where a multiplier exceeds 1, reads the untouched input again and inverts that with partial pivoting
-// there.  One launch of 12 us at N = 36 (9 of the 16 four-pivot steps) where first block, two steps and the check
+// there.  One launch of 9 us at N = 36 (9 of the 16 four-pivot steps) where first block, two steps and the check
 // for the fallback took 28
 __device__ __forceinline__ void gj_small_body(GjLds<64> &sh, double *__restrict__ M, unsigned n, double *__restrict__ diag,
 		int *__restrict__ piv, double *__restrict__ scal)

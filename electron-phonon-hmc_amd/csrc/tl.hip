@@ -1691,8 +1691,7 @@ extern "C" int ephmc_tl_hist(ephmc_ctx *c, const double *normals, unsigned nsamp
 #undef EPHMC_TRIDIAG
 			}else{
 				const size_t lds = (3 * (size_t)n + TL_BT / 64) * 8;
-				if(n <= TL_BT) tl_tridiag_kernel<TL_BT, 1><<<nb_, TL_BT, lds, c->stream>>>(w.A, n, w.d, w.e, w.tau);
-				else tl_tridiag_kernel<TL_BT, 2><<<nb_, TL_BT, lds, c->stream>>>(w.A, n, w.d, w.e, w.tau);
+				tl_tridiag_kernel<TL_BT, 2><<<nb_, TL_BT, lds, c->stream>>>(w.A, n, w.d, w.e, w.tau);
 			}
 			EPHMC_LAUNCHED();
 		}
