@@ -277,7 +277,8 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs<R> &a, unsigned bx, u
 				}
 			}
 		}
-
+		// buf1 was read last, and is the first that S is written to
+		__syncthreads();
 	}
 
 	// ---- W state --------------------------------------------------------------------------
