@@ -145,6 +145,18 @@ int timer_end(ephmc_ctx *c, const char *group)
 	return EPHMC_OK;
 }
 
+__global__ void zero_kernel(double *a, size_t n)
+{
+	for(size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] = 0;
+}
+
+static int set_zero(ephmc_ctx *c, double *a, size_t n)
+{
+	zero_kernel<<<(unsigned)std::min<size_t>((n + 255) / 256, 1024), 256, 0, c->stream>>>(a, n);
+	EPHMC_LAUNCHED();
+	return EPHMC_OK;
+}
+
 // Columns per workgroup of the adjoint sweep.  A slice's partial bond sums (3 N per workgroup) and its
 // coefficients are paid per workgroup, so wide ones win even where they leave CUs idle, until latency is
 // what counts: per 32 slices 16x16 45 us at 1 column and 53 at 2 (fp64); 21x19 110 at 1, 81 at 2, 118 at 4
@@ -447,11 +459,11 @@ int ephmc_create(const ephmc_config *cfg, ephmc_ctx **out)
 		|| hipMemcpy(c->d_link, link.data(), link.size() * sizeof(unsigned), hipMemcpyHostToDevice) != hipSuccess
 		|| hipMemcpy(c->d_twiddle, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess
 		|| hipMemcpy(c->d_f2, f2.data(), f2.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess
-		|| hipMemcpy(c->d_f2mom, f2m.data(), f2m.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess
-		|| hipMemset(c->d_scal, 0, SCAL_COUNT * sizeof(double)) != hipSuccess){
+		|| hipMemcpy(c->d_f2mom, f2m.data(), f2m.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess){
 		set_error("initial uploads failed");
 		return fail(EPHMC_ERR_HIP);
 	}
+	if((rc = set_zero(c, c->d_scal, SCAL_COUNT)) != EPHMC_OK) return fail(rc);
 	if((rc = patch_reserve(c, EPHMC_FP64)) != EPHMC_OK || (mixed && (rc = patch_reserve(c, EPHMC_MIXED)) != EPHMC_OK)) return fail(rc);
 	// the stabilised product's buffers now, so that a captured trajectory allocates nothing
 	if(cfg->stabilize && (rc = stab_reserve(c)) != EPHMC_OK) return fail(rc);
@@ -847,18 +859,6 @@ int ephmc_gj_fallbacks(ephmc_ctx *c, unsigned long *count)
 // fastest of each.  The sweep's partial buffers grow when a narrower width needs more
 // workgroups.  A captured trajectory graph is dropped, to be captured again with the new
 // shapes.  Uses the MD scratch buffers only; call it between trajectories.
-__global__ void zero_kernel(double *a, size_t n)
-{
-	for(size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] = 0;
-}
-
-static int set_zero(ephmc_ctx *c, double *a, size_t n)
-{
-	zero_kernel<<<(unsigned)std::min<size_t>((n + 255) / 256, 1024), 256, 0, c->stream>>>(a, n);
-	EPHMC_LAUNCHED();
-	return EPHMC_OK;
-}
-
 // fastest of reps single runs after one warm-up run (code load): a transient slowdown, such as
 // the clock still rising, costs one sample rather than the average
 static int time_ms(ephmc_ctx *c, hipEvent_t e0, hipEvent_t e1, int reps, double *ms, const std::function<int()> &body)
