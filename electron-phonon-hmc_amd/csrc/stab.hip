@@ -282,7 +282,8 @@ __device__ __forceinline__ void factor_panel(double *__restrict__ z, unsigned n,
 			a[k][q] = z[(size_t)min(j0 + 4 * c4 + k, n - 1) * n + min(j0 + rr, n - 1)];
 			if(4 * c4 + k >= (int)nb || rr >= m) a[k][q] = 0.0;
 		}
-	for(int e = tid; e < NB * NB; e += BT) tl[(e / NB) * LD + e % NB] = 0.0;
+	// T, and V^T V: the sums for T run over all NB columns, of which a panel of nb < NB forms nb
+	for(int e = tid; e < 2 * NB * LD; e += BT) gm[e] = 0.0;
 	int refl = 0;
 #pragma unroll 1
 	for(int jq = 0; jq < NC; jq++)
@@ -374,7 +375,7 @@ __device__ __forceinline__ void factor_panel(double *__restrict__ z, unsigned n,
 	}
 	if(tid == 0) *nref = (first ? 0 : *nref) + refl;
 	__syncthreads();
-	// T: T_jj = t_j (zero past nb: those rows and columns of T stay zero), V^T V = gm
+	// T: T_jj = t_j, V^T V = gm (both zero past nb: those rows and columns of T stay zero)
 	upper_from_diagonal<NB, BT>(gm, tl, tmp);
 	for(int e = tid; e < NB * NB; e += BT) tm[e] = tl[(e / NB) * LD + e % NB];
 }

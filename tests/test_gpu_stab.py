@@ -135,3 +135,26 @@ def test_blocked_qr_sizes(l1, l2, nt, k):
     ld1, s1, inv1 = ctx.stable_logdet_inv(x, 0, k)
     assert s1 == sign and ld1 == pytest.approx(ld, rel=1e-11)
     assert rel(inv1, np.linalg.inv(M).T.ravel()) < 1e-11
+
+
+# N below one panel, and above 1024 sites not a multiple of its 16 columns
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("l1,l2,nt,k", [(1, 1, 4, 1), (5, 5, 8, 3), (13, 2, 8, 4), (41, 25, 8, 4)])
+def test_blocked_qr_reads_no_leftovers(l1, l2, nt, k, precision):
+    """The same values after a kernel that left NaN all over the LDS: a field of NaN through the boson
+    transform (66 KB per workgroup, more workgroups than CUs) before the product.  Against numpy's for
+    the plain FP64 product: 1e-11 as above, and FP32 accuracy with FP32 slices."""
+    dirty = gpu_context(OracleModel(32, 32, 512))
+    nan = np.full(dirty.dim, np.nan)
+    om = OracleModel(l1, l2, nt, beta=4.0)
+    ctx = gpu_context(om, precision=precision)
+    x = np.random.default_rng(l1 + l2).standard_normal(om.dim)
+    n = l1 * l2
+    say("blocked QR after NaN in LDS", l1, l2, nt, k, precision)
+    M = ctx.M_hat(x).reshape(n, n).T
+    sign, ld = np.linalg.slogdet(M)
+    dirty.update_x(nan, nan, 0.1, 1.0)
+    ld1, s1, inv1 = ctx.stable_logdet_inv(x, precision, k)
+    tol = 1e-11 if precision == 0 else 1e-5
+    assert s1 == sign and ld1 == pytest.approx(ld, rel=tol)
+    assert rel(inv1, np.linalg.inv(M).T.ravel()) < tol
