@@ -63,17 +63,18 @@ __global__ void coef_multi_kernel(const CoefArgs *__restrict__ tab)
 	coef_body(a.x, a.link, a.t[0], a.t[1], a.t[2], a.k[0], a.k[1], a.k[2], a.ns, a.nt, a.c64, a.c32, blockIdx.x, a.gx);
 }
 
-// the site form's coefficients (blockIdx.y < nt: slice blockIdx.y) and the patch form's
-// (blockIdx.y - nt: its slice) of one arithmetic, in one launch
+// the site form's coefficients (blockIdx.x < nt: slice blockIdx.x) and the patch form's
+// (blockIdx.x - nt: its slice) of one arithmetic, in one launch.  The slices lie on the grid's first axis,
+// the only one that takes more than 65535 workgroups
 template <typename R>
 __global__ __launch_bounds__(256) void coef_patch_kernel(const double *__restrict__ x, const unsigned *__restrict__ link,
 		double t0, double t1, double t2, double k0, double k1, double k2, unsigned ns, unsigned nt, double *__restrict__ c64,
 		float *__restrict__ c32, const int *__restrict__ bond, unsigned nbond, R *__restrict__ out)
 {
-	const bool site = blockIdx.y < nt;
-	const size_t tau = site ? blockIdx.y : blockIdx.y - nt;
+	const bool site = blockIdx.x < nt;
+	const size_t tau = site ? blockIdx.x : blockIdx.x - nt;
 	const unsigned n = site ? 6 * ns : nbond;
-	for(unsigned e = blockIdx.x * 256 + threadIdx.x; e < n; e += gridDim.x * 256){
+	for(unsigned e = blockIdx.y * 256 + threadIdx.x; e < n; e += gridDim.y * 256){
 		const int b = site ? (int)link[e] : bond[e], k = b % 3;
 		const double tk = k == 0 ? t0 : (k == 1 ? t1 : t2);
 		const double kk = k == 0 ? k0 : (k == 1 ? k1 : k2);
@@ -94,7 +95,7 @@ int coefficients(ephmc_ctx *c, const double *x, bool want32)
 	if(patch_on(c, want32 ? EPHMC_MIXED : EPHMC_FP64)){
 		c->patch_slot = want32 ? 1 : 0;
 		const unsigned m = pt.nk * pt.tp;
-		const dim3 g((std::max(m, 6 * c->ns) + 255) / 256, 2 * c->nt);
+		const dim3 g(2 * c->nt, (std::max(m, 6 * c->ns) + 255) / 256);
 		if(want32) coef_patch_kernel<float><<<g, 256, 0, c->stream>>>(x, c->d_link, t[0], t[1], t[2], k[0], k[1], k[2], c->ns, c->nt,
 			c->d_coef64, c32, pt.bond, m, (float *)pt.coef);
 		else coef_patch_kernel<double><<<g, 256, 0, c->stream>>>(x, c->d_link, t[0], t[1], t[2], k[0], k[1], k[2], c->ns, c->nt,

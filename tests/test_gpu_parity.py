@@ -508,3 +508,18 @@ def test_force_sweep_columns(l1, l2, nt, order, prec, monkeypatch):
                 continue
             assert rel(bits[-1], ref) < tol
             np.testing.assert_array_equal(bits[-1], bits[0])
+
+
+def test_more_slices_than_a_grid_axis():
+    """40000 slices: 80000 rows of coefficients, beyond the 65535 workgroups of a grid's second axis.
+    M_hat, log det and force against the oracle; each slice rounds by about 10 eps at most, so 1e-10
+    for the product and 1e-9 for the force, which multiplies two such products with the inverse."""
+    om = OracleModel(3, 2, 40000)
+    ctx = gpu_context(om, checkpoint=0)
+    x = np.random.default_rng(4).standard_normal(om.dim)
+    say("40000 slices")
+    M = om.M_hat(x)
+    assert rel(ctx.M_hat(x), M) < 1e-10
+    ld, _, inv = om.logdet_inv(M)
+    assert ctx.logdet_inv(M)[0] == pytest.approx(ld, rel=1e-10)
+    assert rel(ctx.force(x, inv, ld), om.force(x, inv, ld)) < 1e-9
