@@ -979,10 +979,8 @@ int ephmc_autotune(ephmc_ctx *c, ephmc_tune_result *res)
 			if(sh.ms < ms_out){ ms_out = sh.ms; cols_out = sh.C; strip_out = sh.M; }
 		c->chain_cols_set[slot] = cols_out;
 		c->chain_strip_set[slot] = cols_out ? (int)strip_out : -1;
-		if(cols_out == 0){
-			cols_out = c->patch[slot].cols;
-			strip_out = c->patch[slot].px == 2 && c->l1 % 2 == 0 ? 2 : 0;
-		}
+		// the patch form reports its columns and no strip: a strip of 2 would name another, slower form
+		if(cols_out == 0) cols_out = c->patch[slot].cols;
 		return EPHMC_OK;
 	};
 	do {
