@@ -706,7 +706,8 @@ __global__ __launch_bounds__(1024) void tl_bisect_kernel(const double4 *__restri
 // T - x but row r, which leaves gamma_r: r is where |gamma| is smallest.  Each relation is local, so
 // rounding leaves a residual of eps |T| in every row whatever the pivots' size; a pivot below
 // 2^-52 is moved there, a change of d by as much.  l, u and z: [i][k], lanes on consecutive k.
-// rn = 1 / |z|.  A residual above 1e-13 sends the sample to the QL iteration.
+// rn = 1 / |z|.  A residual above 2^-47 of the norm (they reach 4e-16 at N = 36, 8e-16 at 256, 1.4e-15 at 1024),
+// or a vector that overflowed, sends the sample to the QL iteration.
 __global__ __launch_bounds__(256) void tl_vectors_kernel(const double4 *__restrict__ tsall, const double *__restrict__ tn,
 		const double *__restrict__ evall, unsigned n, double *__restrict__ lu, size_t lu_stride, double *__restrict__ Zall,
 		double *__restrict__ rnall, int *__restrict__ ql)
@@ -761,11 +762,13 @@ __global__ __launch_bounds__(256) void tl_vectors_kernel(const double4 *__restri
 	}
 	const double rn = 1.0 / sqrt(ss);
 	rnall[(size_t)s * n + k] = rn;
-	if(!(best * rn < 1e-13)) ql[s] = 1;
+	if(!(best * rn < 0x1p-47 && rn > 0)) ql[s] = 1;
 }
 
 // Vectors whose eigenvalues differ by less than 2^-14 of the norm, made orthogonal one after the other
-// within each run of such neighbours (beyond it eps / gap bounds the overlap by 4e-12).  Of a run's
+// within each run of such neighbours.  Beyond it the residuals' sum over the gap bounds an overlap, by 2^-32
+// for residuals of 2^-47; those met leave 3e-12 at N = 1024, with bins no further
+// from 64-bit ones than the QL iteration's: 1.5e-15 against 4.2e-15 for 1024 samples at N = 256.  Of a run's
 // space any orthonormal basis serves: the pairs it forms share their bins to 2^-14 of the norm and
 // their weights' sum does not depend on the basis.  Vectors that nearly coincide (overlap above 0.85),
 // or a run of more than 16, send the sample to the QL iteration.
