@@ -162,14 +162,17 @@ static int set_zero(ephmc_ctx *c, double *a, size_t n)
 // what counts: per 32 slices 16x16 45 us at 1 column and 53 at 2 (fp64); 21x19 110 at 1, 81 at 2, 118 at 4
 // (fp32 72, 61, 78); 24x24 235 at 2, 194 at 4 (fp32 140, 106); 32x32 334 at 2, 262 at 4 (fp32 173, 126).  Beyond
 // 1024 sites a thread holds two and registers for two columns: 36x36 in fp32 332 at 2, 560 at 4.
+// So they do in fp64 at Taylor orders 6 and 8, whose S spill at four: 24x24 at order 8 456 at 2, 690 at 4,
+// at order 6 295 and 293, 32x32 490 and 849, 326 and 407.
 // EPHMC_ADJOINT_COLS overrides it for tuning sweeps.
-static unsigned adjoint_cols_auto(unsigned ns, int prec)
+static unsigned adjoint_cols_auto(unsigned ns, int prec, int deg)
 {
 	if(const char *e = getenv("EPHMC_ADJOINT_COLS")){
 		const unsigned v = (unsigned)atoi(e);
 		if(v == 1 || v == 2 || v == 4) return v;
 	}
-	for(unsigned C = ns <= 256 ? 1 : ns <= 512 || ns > 1024 ? 2 : 4; C > 1; C >>= 1)
+	const bool two = ns <= 512 || ns > 1024 || (prec == EPHMC_FP64 && deg > 4);
+	for(unsigned C = ns <= 256 ? 1 : two ? 2 : 4; C > 1; C >>= 1)
 		if(adjoint_lds(ns, prec, C) <= 160 * 1024) return C;
 	return 1;
 }
@@ -399,7 +402,7 @@ int ephmc_create(const ephmc_config *cfg, ephmc_ctx **out)
 	else c->ckpt = (size_t)c->nt * c->mat * rsz <= ((size_t)4 << 30) ? 1u : std::min(16u, c->nt);
 	c->nseg = (c->nt + c->ckpt - 1) / c->ckpt;
 	c->span = c->ckpt == 1 ? std::min(32u, c->nt) : c->ckpt;
-	c->cols = adjoint_cols_auto(ns, cfg->precision);
+	c->cols = adjoint_cols_auto(ns, cfg->precision, c->poly.deg);
 	c->adj_w0_early = 1;
 	if(const char *e = getenv("EPHMC_ADJOINT_W0EARLY")) c->adj_w0_early = atoi(e) != 0;
 	c->nwg = (ns + c->cols - 1) / c->cols;

@@ -523,3 +523,21 @@ def test_more_slices_than_a_grid_axis():
     ld, _, inv = om.logdet_inv(M)
     assert ctx.logdet_inv(M)[0] == pytest.approx(ld, rel=1e-10)
     assert rel(ctx.force(x, inv, ld), om.force(x, inv, ld)) < 1e-9
+
+
+@pytest.mark.parametrize("l1,l2", [(24, 24), (32, 32)])
+@pytest.mark.parametrize("taylor", [6, 8])
+def test_force_sweep_width_of_high_orders(l1, l2, taylor, monkeypatch):
+    """FP64 sweeps of Taylor orders 6 and 8 take two columns per workgroup between 513 and 1024 sites (four
+    spill: 24x24 at order 8 690 against 456 us per 32 slices): the same bits as with two asked for, which
+    group the partial sums unlike four."""
+    om = OracleModel(l1, l2, 4, beta=5.0, taylor=taylor)
+    x = np.random.default_rng(taylor).standard_normal(om.dim)
+    say("sweep width", l1, l2, taylor)
+    force = {}
+    for cols in (None, "2", "4"):
+        if cols:
+            monkeypatch.setenv("EPHMC_ADJOINT_COLS", cols)
+        force[cols] = gpu_context(om, checkpoint=0, taylor_order=taylor).md_force(x)
+    np.testing.assert_array_equal(force[None], force["2"])
+    assert not np.array_equal(force[None], force["4"])
