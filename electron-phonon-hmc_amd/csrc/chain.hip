@@ -542,7 +542,10 @@ static int launch_patch(ephmc_ctx *c, const PatchTab &t, PatchArgs<R> a)
 // shapes above): fp64 up to 512 sites one site per thread and one column per workgroup, above 640
 // sites 2 x 2 sites and 2 columns (between, the strip form by 3 % where l1 is even); fp32 not up to
 // 256 sites (16x16 nt 64: 62 against 55 us for the site form), one site and 2 columns up to 640, 2 x 2
-// sites and 2 columns beyond.
+// sites and 2 columns beyond.  Not 2 x 2 where the lattice is one site wide, as half of a patch would be ghosts
+// (fp64 1x1024 nt 32 200 us against 120 for the site form, 1500x1 431 against 277 for strips; fp32 1x1024 108
+// against 83), nor in fp64 over strips where a quarter would (400x3 273 against 236; 300x5, with a sixth, 292
+// against 288; where l1 is odd, patches stay the faster: 3x400 276 against 293).
 int patch_reserve(ephmc_ctx *c, int prec)
 {
 	PatchTab &t = c->patch[prec == EPHMC_FP64 ? 0 : 1];
@@ -554,6 +557,8 @@ int patch_reserve(ephmc_ctx *c, int prec)
 	t.px = X; t.py = Y;
 	t.npx = (c->l1 + X - 1) / X;
 	t.np = t.npx * ((c->l2 + Y - 1) / Y);
+	const bool strips = prec == EPHMC_FP64 && c->l1 % 2 == 0;
+	if(X == 2 && (c->l1 == 1 || c->l2 == 1 || (strips && 16 * t.np > 5 * ns))){ t = PatchTab{}; return EPHMC_OK; }
 	t.tp = (t.np + 63) / 64 * 64;
 	if(t.tp > 1024){ t = PatchTab{}; return EPHMC_OK; }        // (long thin lattices)
 	t.nk = patch_bonds(X, Y);
