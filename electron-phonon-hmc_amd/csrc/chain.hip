@@ -559,8 +559,7 @@ int patch_reserve(ephmc_ctx *c, int prec)
 	t.np = t.npx * ((c->l2 + Y - 1) / Y);
 	const bool strips = prec == EPHMC_FP64 && c->l1 % 2 == 0;
 	if(X == 2 && (c->l1 == 1 || c->l2 == 1 || (strips && 16 * t.np > 5 * ns))){ t = PatchTab{}; return EPHMC_OK; }
-	t.tp = (t.np + 63) / 64 * 64;
-	if(t.tp > 1024){ t = PatchTab{}; return EPHMC_OK; }        // (long thin lattices)
+	t.tp = (t.np + 63) / 64 * 64;               // at most 704 (3 x 680 sites)
 	t.nk = patch_bonds(X, Y);
 	const unsigned nh = patch_halo(X, Y), tp = t.tp;
 	std::vector<int> tab((size_t)(nh + t.nk) * tp, 0);
