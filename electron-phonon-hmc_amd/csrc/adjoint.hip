@@ -23,7 +23,7 @@
 // 256 sites (512 in fp64) their latency bounds the sweep, so the next slice's S is built under this
 // slice's W phases: deg barriers a slice instead of 2 deg - 1, 32 slices of 6x6 38.5 -> 34.9 us, 64 of
 // 16x16 56.4 -> 45.4.  With 1024 threads registers are what is short: 32 slices of 32x32 in fp64 at four
-// columns 340 -> 262 us, of 36x36 at two 1721 -> 1209 (no more spills in the loop), in fp32 134 -> 128; there a
+// columns 340 -> 262 us, of 36x36 at two 1721 -> 1209 (44 registers spilled instead of 63), in fp32 134 -> 128; there a
 // workgroup's reads of LDS take 4.5 of the 8 us per slice in fp64, 2.2 of 4 in fp32, and T and the partial sums
 // about as long at the rate of memory.
 #include "internal.h"

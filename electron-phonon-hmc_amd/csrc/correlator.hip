@@ -14,7 +14,7 @@
 //   g_ab(tau) = -1/N sum_{i,j} (J_a R_t0)[i][j] (J'_b Q)[j][i]:
 // two neighbours of i in R_t0's column j per a, two neighbours of j in Q's rows per b, then nine
 // products, in place of four products of gathered entries for each of the nine (a, b).
-// One launch covers every tau.  A workgroup takes up to CC_L sites j of a lattice row (of CC_R rows
+// One launch covers every tau.  A workgroup takes up to CC_L sites j of a lattice row (of several rows
 // where rows are short) and walks them in order: R_t0's column goes through LDS for the neighbours in
 // i, the rows of Q slide along in registers (three new ones per j), all loaded one j ahead.  Block
 // sums per (tau, workgroup), then a fixed-order pass per tau.
@@ -73,7 +73,8 @@ __device__ __forceinline__ double cc_diff(double a, double b, double c, double d
 	return a * b - c * d;
 }
 
-// Thread t takes the sites i = t + BT q, q < S (BT S >= N).  Workgroup b: slice and item by cc_item.
+// Thread t takes the sites i = t + BT q, q < S (BT S >= N).  Workgroup b works on item `item` of slice tau, eight
+// slices at a time, one to an XCD.
 // What bounds it: the 2 nt N^2 values read from memory once (2 GB at 32x32, nt 128); each piece's first and
 // last columns and the rows above and below it come a second and third time, from the XCD's L2, to
 // which all workgroups of a slice go.  585 us there, 3.6 TB/s; with the gathered entries of all nine

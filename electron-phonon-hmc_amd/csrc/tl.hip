@@ -19,7 +19,8 @@
 //                   rank-2 update of step j fused with the matrix-vector product of step j+1
 //                   (read and written once per step).  Reflectors v_j overwrite column j below
 //                   the diagonal.
-//   tl_bisect       (3 <= N <= 1024) eigenvalues by bisection with Sturm counts, one per thread
+//   tl_bisect       (N = 27 .. 34 and 42 .. 1024, where tl_back's panels fit the rotations' buffer) eigenvalues
+//                   by bisection with Sturm counts, one per thread
 //   tl_vectors      eigenvectors of the tridiagonal matrix by twisted factorisation, one per thread;
 //                   tl_orthogonalise makes neighbours with a small gap orthogonal.  A sample where
 //                   that does not hold (eigenvalues equal to rounding) takes the QL iteration below,
@@ -31,12 +32,12 @@
 //                   pass with a register window of G+1 columns (a wavefront: sweep g runs one
 //                   position behind sweep g-1), so Z is read and written once per G sweeps;
 //                   columns are loaded several steps ahead
-//   tl_back         V = H_0 H_1 ... H_{N-3} Z in compact-WY blocks of 32 reflectors (N <= 1024):
+//   tl_back         V = H_0 H_1 ... H_{N-3} Z in compact-WY blocks of 32 reflectors (the same N):
 //                   tl_yb (each block's reflectors as a row-major N x 32 panel) and tl_wy_t (the
 //                   blocks' T factors), then
 //                   tl_wy_apply, a workgroup per 16 columns of Z held in matrix-core accumulators
 //                   for the whole sweep (Z <- Z - Y (T (Y^T Z)) per block, last block first);
-//                   larger N: a wave holds CW columns of Z in registers and applies every
+//                   other N: a wave holds CW columns of Z in registers and applies every
 //                   reflector (last first)
 //   tl_sort         eigenvalue ranks, e^{-E}, the partition sum
 //   tl_current      V sorted by eigenvalue and W_c = G_c V (gather form of the bond currents)
@@ -1700,7 +1701,8 @@ extern "C" int ephmc_tl_hist(ephmc_ctx *c, const double *normals, unsigned nsamp
 		}
 		EPHMC_TRY(timer_end(c, "tl_tridiag"));
 		// back-transformation in compact-WY blocks on the matrix cores (N <= 1024), the reflector copy and
-		// the T factors in the rotation buffer, which is free by then; else one reflector at a time
+		// the T factors in the rotation buffer, which is free by then; else one reflector at a time.  The buffer
+		// holds 1.5 N^2 rotations: too few for the padded panels of N = 3 .. 26 and 35 .. 41
 		const unsigned nblkw = n > 2 ? (n - 2 + TL_WB - 1) / TL_WB : 0;
 		const size_t ybsz = (size_t)nblkw * ((n + 15) & ~15u) * TL_WB;
 		const bool wy = n >= 3 && n <= TL_WW * 16 * TL_WRB && ybsz + (size_t)nblkw * TL_WB * TL_WB <= 2 * w.rot_cap;

@@ -179,3 +179,11 @@ def test_tl_many_samples_repeatable(l1, l2):
     for q in range(ns - 8, ns):
         E = np.linalg.eigvalsh(D.hopping_matrix(om.nnt, om.ns, xs[q], om.t, om.kappa, -om.mu))
         assert abs(runs[0][1][q] / (np.exp(-E).sum() / om.ns) - 1) < 1e-12
+
+
+@pytest.mark.parametrize("l1,l2", [(9, 3), (17, 2), (7, 6)])
+@pytest.mark.parametrize("scale", [0.0, 1e-9, 1e-4, 1e-2])
+def test_tl_degenerate_pairs_smallest(l1, l2, scale):
+    """test_tl_degenerate_pairs at the smallest lattices whose eigenvalues come from bisection (27 .. 34 and
+    from 42 sites on; 3 x 3 and 6 x 6 take the QL iteration)."""
+    test_tl_degenerate_pairs(l1, l2, scale)
